@@ -83,9 +83,14 @@ struct BwK {
   int tb;                 // tokens per tile: 4, or 2 (two-token tiles; n_tiles counts those)
   int xb;                 // 4-token tiles of raw bf16 (8-byte slots; bf16 X)
   int wbf;                // W and bias stored as bf16 (widened in the kernel)
+  int tps;                // window staging: tiles per stage (WS_TILES for pool windows)
   const uint16_t* fm;     // the forward's ReLU bits ([n_chunks][fm_tiles][64] 16-bit words) or null
   int fm_tiles, fm_t0;    // 4-token tiles of the whole batch; the backward chunk's first tile
 };
+
+// 16-byte slots of one stage region of the dW pass over narrow layers: two regions in 50 KiB, three
+// workgroups per CU
+constexpr int BWD_WS_SMALL = 1600;
 
 // One token tile of the dW pass (LDS at xsb): recompute z, form dz = c1 * act'(z), accumulate
 // db, dW and the tile's 4 mask bits (bit 4 (t % 8) + i of word mw for token i of tile t).  The
@@ -267,7 +272,7 @@ __device__ __forceinline__ void bwd_w_tile2(const char* xsb, int t, const float2
 // c1 row are addressed with scalar registers.
 template <int K, int NPL, int WAVES, int ACT, int RA, bool DBUF, bool WS = false, bool XG = false, int TB = BT,
           bool XB = false, bool FM = false, bool SMALL = false>
-__global__ void __launch_bounds__(WAVES * 64, SMALL ? 4 : 1) bwd_w_kernel(BwK p) {
+__global__ void __launch_bounds__(WAVES * 64, SMALL ? (WS ? 3 : 4) : 1) bwd_w_kernel(BwK p) {
   // XG (D > XTILE_SB): no LDS tile, the lanes gather from the token tiles in global memory.
   // TB: tokens per tile, 4 or 2 (two-token tiles in the two buffers of DBUF: D <= 2 XTILE_DB)
   static_assert(TB == BT || (TB == 2 && DBUF && !WS && !XG), "two-token tiles: double-buffered only");
@@ -275,11 +280,12 @@ __global__ void __launch_bounds__(WAVES * 64, SMALL ? 4 : 1) bwd_w_kernel(BwK p)
   // staged from them
   static_assert(!XB || (TB == BT && (DBUF || SMALL || WS) && !XG), "bf16 tiles: double- or small-buffered, windows");
   // SMALL: one single-buffered 64-KiB tile per workgroup, two workgroups per CU (128 VGPRs at most)
-  static_assert(!SMALL || (!DBUF && !WS && !XG && TB == BT), "small: one 4-token tile per workgroup");
+  // SMALL with WS: stages of narrow tiles in a third of the LDS, three workgroups per CU
+  static_assert(!SMALL || (!DBUF && !XG && TB == BT), "small: one 4-token tile per workgroup");
   // FM: the mask bits come from the forward (p.fm): no z recompute, W and bias are not read
   static_assert(!FM || (TB == BT && ACT == GL_ACT_RELU), "forward ReLU bits: 4-token tiles, ReLU");
   constexpr unsigned SLOT = XB ? 8u : 4u * TB;  // bytes per input of a tile
-  __shared__ float4 xs[DBUF || WS ? 2 * XTILE_DB : (XG ? 1 : (SMALL ? XTILE_DB : XTILE_SB))];
+  __shared__ float4 xs[WS && SMALL ? 2 * BWD_WS_SMALL : DBUF || WS ? 2 * XTILE_DB : (XG ? 1 : (SMALL ? XTILE_DB : XTILE_SB))];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   long long chunk = (long long)blockIdx.x * WAVES + wave;
@@ -296,8 +302,9 @@ __global__ void __launch_bounds__(WAVES * 64, SMALL ? 4 : 1) bwd_w_kernel(BwK p)
   unsigned slot2[(NPL + 1) / 2];  // slots of neurons 2i, 2i+1 within the pool (16 bits each; >= n_g: padding)
   // window staging: this wave's pool is slot pk of the workgroup's staged pools, window start lo
   const int g_first = (int)((long long)blockIdx.x * WAVES / p.cpg);
-  const int pk = WS ? (int)(g - g_first) : 0;
-  const int lo = WS ? (int)__builtin_amdgcn_readfirstlane(p.win[g]) : 0;
+  // (whole tiles staged, p.win null: one window of all inputs)
+  const int pk = WS && p.win ? (int)(g - g_first) : 0;
+  const int lo = WS && p.win ? (int)__builtin_amdgcn_readfirstlane(p.win[g]) : 0;
   // the lane's neurons: LDS addresses of their inputs, weights, bias, slots
   if constexpr (WS) {
     // pool windows: the parameter dtype tested per load (the set-up below, written as a generic
@@ -376,13 +383,14 @@ __global__ void __launch_bounds__(WAVES * 64, SMALL ? 4 : 1) bwd_w_kernel(BwK p)
   constexpr int TPW = 32 / TB;       // tiles per mask word
   const int ns = (int)((long long)p.D * SLOT / 16);  // 16-byte slots per tile (D even for 8-byte slots)
 
-  // window staging: WS_TILES tiles per stage and barrier; tile t at slot (t mod 2 WS_TILES) * nsl
+  // window staging: tps tiles per stage and barrier; tile t at slot (t mod 2 tps) * nsl
+  const int tps = p.tps;
   const WinLayout L{p.win, p.ww, p.npw, g_first, p.G};
   const int nsl = p.npw * p.ww;
   const unsigned tstep = (unsigned)nsl * SLOT;
-  const int rslots = WS_TILES * nsl * (int)SLOT / 16;  // 16-byte slots per stage region
+  const int rslots = tps * nsl * (int)SLOT / 16;  // 16-byte slots per stage region
   if constexpr (WS) {
-    dma_window_stage<SLOT>(p.xt, xs, 0, p.n_tiles, p.D, L, WAVES);
+    dma_stage<SLOT>(p.xt, xs, 0, tps, p.n_tiles, p.D, L, WAVES);
     stage_wait();
     __syncthreads();
   } else if constexpr (DBUF) {
@@ -408,12 +416,12 @@ __global__ void __launch_bounds__(WAVES * 64, SMALL ? 4 : 1) bwd_w_kernel(BwK p)
     for (int j = 0; j < NPL; ++j) mw[j] = 0u;
     const int t1 = t0 + TPW < p.n_tiles ? t0 + TPW : p.n_tiles;
     if constexpr (WS) {
-      for (int ts0 = t0; ts0 < t1; ts0 += WS_TILES) {
-        const int r = (ts0 / WS_TILES) & 1;
+      for (int ts0 = t0; ts0 < t1; ts0 += tps) {
+        const int r = (ts0 & tps) ? 1 : 0;
         // region r ^ 1 was last read in the previous stage, which every wave finished before the barrier
-        if (ts0 + WS_TILES < p.n_tiles)
-          dma_window_stage<SLOT>(p.xt, xs + (r ^ 1) * rslots, ts0 + WS_TILES, p.n_tiles, p.D, L, WAVES);
-        const int tn = p.n_tiles - ts0 < WS_TILES ? p.n_tiles - ts0 : WS_TILES;
+        if (ts0 + tps < p.n_tiles)
+          dma_stage<SLOT>(p.xt, xs + (r ^ 1) * rslots, ts0 + tps, tps, p.n_tiles, p.D, L, WAVES);
+        const int tn = p.n_tiles - ts0 < tps ? p.n_tiles - ts0 : tps;
         for (int tt = 0; tt < tn; ++tt) {
           const int t = ts0 + tt;
           const float4 c1 = ld_uniform4(c1row, t * BT);
@@ -424,7 +432,7 @@ __global__ void __launch_bounds__(WAVES * 64, SMALL ? 4 : 1) bwd_w_kernel(BwK p)
             bwd_w_tile<K, NPL, ACT, RA, false, const char*, FM>(reinterpret_cast<const char*>(xs), t, c1, addr, w, bias,
                                                                dw, dbv, mw, fbits(t));
           // next tile's slot; after the last tile of region 1 back to region 0 (uniform step, no branch)
-          const unsigned step = (t & (2 * WS_TILES - 1)) == 2 * WS_TILES - 1 ? tstep - 2u * WS_TILES * tstep : tstep;
+          const unsigned step = (t & (2 * tps - 1)) == 2 * tps - 1 ? tstep - 2u * (unsigned)tps * tstep : tstep;
 #pragma unroll
           for (int j = 0; j < NPL; ++j)
 #pragma unroll
@@ -1635,6 +1643,19 @@ void edge_layout(int D, int G, int S, int K, EdgeHeader* h, size_t* total) {
 
 template <int K, int NPL, int WAVES, int ACT, int RA>
 static int launch_bwd_w(const BwK& k, hipStream_t s) {
+  if constexpr (K == 8)
+    if (k.tps && !k.win) {
+      // 12 waves per CU as the wide kernel's, but a barrier holds 4 of them, not 12, the next stage
+      // loads meanwhile, and small layers spread over the CUs in thirds.  One 12-wave workgroup ->
+      // this: 1M neurons, 64 tokens, D = 1024 159 -> 116 us; 4M, 256 tokens D = 1024 1180 -> 905,
+      // D = 200 1169 -> 747; 1M, D = 1500 152 -> 112.  The same stages in one 12-wave workgroup
+      // 1118 / 1053.  Not at fan-in 16 (the 2-neuron kernel needs 188 VGPRs: 169 -> 245 us).
+      constexpr int W = 4;
+      auto fs = bwd_w_kernel<K, NPL, W, ACT, RA, false, true, false, BT, false, false, true>;
+      GL_LAUNCH(GL_KERNEL_BWD_W, fs, dim3((unsigned)ceil_div(k.n_chunks, W)), dim3(W * 64), 0, s, k);
+      GL_CHECK_LAUNCH();
+      return 0;
+    }
   auto fn = k.win ? (k.xb ? bwd_w_kernel<K, NPL, WAVES, ACT, RA, false, true, false, BT, true>
                           : bwd_w_kernel<K, NPL, WAVES, ACT, RA, false, true>)
                   : k.xb ? bwd_w_kernel<K, NPL, WAVES, ACT, RA, true, false, false, BT, true>
@@ -1926,7 +1947,11 @@ extern "C" int gl_bwd(const GlBwdArgs* a, void* stream) {
            a->D, a->S, q.cpg, n_tiles * BT / tb, cap, 2 * T, ceil_div(a->S, SCHED_WIN), a->G, ww, npw, a->rec_shift,
            sps, gs, tb, xb ? 1 : 0};
     bk.wbf = wbf;
-    if (win) bk.win = a->win;
+    if (win) bk.win = a->win, bk.tps = WS_TILES;
+    // narrow layers at fan-in 8 (a tile of at most BWD_WS_SMALL inputs): stages of whole tiles in
+    // workgroups of 4 waves, three per CU
+    if (!win && !a->relu_mask && a->K == 8 && a->D <= BWD_WS_SMALL)
+      bk.tps = stage_tiles(a->D, 16, BWD_WS_SMALL, n_tiles), bk.ww = a->D, bk.npw = 1;
     if (a->relu_mask) {  // the forward's bits, per 4-token tile of the batch
       if (tb != BT) return GL_ERR_ARG;
       bk.fm = (const uint16_t*)a->relu_mask;

@@ -230,6 +230,19 @@ struct WinLayout {
   int ww, npw, g_first, G;
 };
 
+// Narrow layers stage whole token tiles the same way: with win null the "window" is the tile (lo = 0,
+// ww = D, one for every pool), and a stage is tps tiles, contiguous in memory.  tps is the largest
+// power of two (at most 8, the tiles of a mask word) whose tiles fit a region of `slots` 16-byte
+// slots, and no more than a pass has tiles; 0 when not even one tile fits.
+inline int stage_tiles(int D, int in_bytes, int slots, int n_tiles) {
+  int tps = 0;
+  for (int t = 1; t <= 8 && (long long)t * D * in_bytes <= (long long)slots * 16; t *= 2) {
+    if (tps >= n_tiles) break;
+    tps = t;
+  }
+  return tps;
+}
+
 // region <- the WS_TILES tiles from t0 (tiles past n_tiles repeat the last one: in bounds, unread).
 // A stage is WS_TILES * npw runs (one tile's window of one pool, ww slots); wave w copies runs
 // w, w + waves, ...  (taking its own runs directly: walking every 64-slot group of the stage in
@@ -260,6 +273,17 @@ __device__ __forceinline__ void dma_window_stage(const float4* __restrict__ xt, 
       asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %2"
                    :: "v"((unsigned)col * 16u), "s"(m0v), "s"(sb) : "memory", "m0");
     }
+  }
+}
+// region <- the tiles [t0, t0 + tps) of n_tiles: pool windows (win), or whole tiles of D inputs
+template <int IB = 16>
+__device__ __forceinline__ void dma_stage(const float4* __restrict__ xt, float4* region, int t0, int tps, int n_tiles,
+                                          int D, const WinLayout& L, int waves) {
+  if (L.win) {
+    dma_window_stage<IB>(xt, region, t0, n_tiles, D, L, waves);
+  } else {
+    const int ns = D * IB / 16;  // 16-byte slots per tile
+    dma_tile(xt + (size_t)t0 * ns, region, (n_tiles - t0 < tps ? n_tiles - t0 : tps) * ns, waves * 64);
   }
 }
 // LDS byte address of input d of a neuron in pool slot k of the workgroup whose window starts at lo

@@ -105,6 +105,7 @@ struct FwdK {
   int pint;               // power mean: p when it is 1, 2, 4 or 8 (exact products), else 0
   int sps, gs;            // pool geometry (pool_base): shards per group and group stride in slots
   int tb;                 // tokens per tile: 4, or 2 (two-token tiles; n_tiles counts those)
+  int tps;                // window staging: tiles per stage (WS_TILES for pool windows)
   int ws_small;           // window staging in workgroups of half the waves (two per CU, 64 KiB of stages)
   int xb;                 // 4-token tiles of raw bf16 (8-byte slots; bf16 X, sum / mean)
   int wbf;                // W and bias stored as bf16 (widened in the kernel)
@@ -824,8 +825,9 @@ __global__ void __launch_bounds__(WAVES * 64, SMALL ? 16 / WAVES * WAVES / 4 : 1
   unsigned vmask = 0u;  // smooth pools: bit j set when neuron j is a valid slot
   // window staging: this wave's pool is slot pk of the workgroup's staged pools, window start lo
   const int g_first = (int)((long long)blockIdx.x * WAVES / p.cpg);
-  const int pk = WS ? (int)(g - g_first) : 0;
-  const int lo = WS ? (int)__builtin_amdgcn_readfirstlane(p.win[g]) : 0;
+  // (whole tiles staged, p.win null: one window of all inputs)
+  const int pk = WS && p.win ? (int)(g - g_first) : 0;
+  const int lo = WS && p.win ? (int)__builtin_amdgcn_readfirstlane(p.win[g]) : 0;
   // the lane's neurons: input addresses, weights, bias, slots
   if constexpr (WS) {
     // pool windows: the parameter dtype tested per load (the set-up below, written as a generic
@@ -902,21 +904,22 @@ __global__ void __launch_bounds__(WAVES * 64, SMALL ? 16 / WAVES * WAVES / 4 : 1
     }
   };
   if constexpr (WS) {
-    // window staging: WS_TILES tiles per stage and barrier; tile t at input (t mod 2 WS_TILES) * nsl
-    // of the stage regions (IB bytes per input)
+    // window staging: tps tiles per stage and barrier; tile t at input (t mod 2 tps) * nsl of the
+    // stage regions (SLOT bytes per input)
+    const int tps = p.tps;
     const WinLayout L{p.win, p.ww, p.npw, g_first, p.G};
     const int nsl = p.npw * p.ww;
     const unsigned tstep = (unsigned)nsl * (unsigned)SLOT;
-    const int rslots = WS_TILES * nsl * (int)SLOT / 16;  // 16-byte slots per region
-    dma_window_stage<SLOT>(p.xt, xa, 0, p.n_tiles, p.D, L, WAVES);
+    const int rslots = tps * nsl * (int)SLOT / 16;  // 16-byte slots per region
+    dma_stage<SLOT>(p.xt, xa, 0, tps, p.n_tiles, p.D, L, WAVES);
     stage_wait();
     __syncthreads();
-    for (int t0 = 0; t0 < p.n_tiles; t0 += WS_TILES) {
-      const int r = (t0 / WS_TILES) & 1;
+    int r = 0;  // the region of the stage being read
+    for (int t0 = 0; t0 < p.n_tiles; t0 += tps, r ^= 1) {
       // region r ^ 1 was last read in the previous stage, which every wave finished before the barrier
-      if (t0 + WS_TILES < p.n_tiles)
-        dma_window_stage<SLOT>(p.xt, xa + (r ^ 1) * rslots, t0 + WS_TILES, p.n_tiles, p.D, L, WAVES);
-      const int tn = p.n_tiles - t0 < WS_TILES ? p.n_tiles - t0 : WS_TILES;
+      if (t0 + tps < p.n_tiles)
+        dma_stage<SLOT>(p.xt, xa + (r ^ 1) * rslots, t0 + tps, tps, p.n_tiles, p.D, L, WAVES);
+      const int tn = p.n_tiles - t0 < tps ? p.n_tiles - t0 : tps;
       for (int tt = 0; tt < tn; ++tt) {
         const int t = t0 + tt;
         if constexpr (XB)
@@ -927,7 +930,7 @@ __global__ void __launch_bounds__(WAVES * 64, SMALL ? 16 / WAVES * WAVES / 4 : 1
                                                     out + t * BT * kp, oslot + t * BT * kp, kp, store, lane, p, mb);
         bits_done(t);
         // next tile's slot; after the last tile of region 1 back to region 0
-        const unsigned step = (t & (2 * WS_TILES - 1)) == 2 * WS_TILES - 1 ? tstep - 2u * WS_TILES * tstep : tstep;
+        const unsigned step = (t & (2 * tps - 1)) == 2 * tps - 1 ? tstep - 2u * (unsigned)tps * tstep : tstep;
 #pragma unroll
         for (int j = 0; j < NPL; ++j)
 #pragma unroll
@@ -1307,7 +1310,7 @@ static int launch_fwd(const FwdK& k, hipStream_t s) {
   if constexpr (PK == PK_SUM && ACT == GL_ACT_RELU && K == 8 && TB == BT)
     if (k.fm) fn = fwd_kernel<K, NPL, WAVES, ACT, DBUF, WS, PK, XG, SMALL, TB, XB, true>;
   dim3 grid((unsigned)ceil_div(k.n_chunks, WAVES));
-  GL_LAUNCH(WS ? GL_KERNEL_FWD_WIN : GL_KERNEL_FWD, fn, grid, dim3(WAVES * 64), 0, s, k);
+  GL_LAUNCH(WS && k.win ? GL_KERNEL_FWD_WIN : GL_KERNEL_FWD, fn, grid, dim3(WAVES * 64), 0, s, k);
   GL_CHECK_LAUNCH();
   return 0;
 }
@@ -1318,7 +1321,7 @@ static int launch_fwd(const FwdK& k, hipStream_t s) {
 template <int ACT, int K, int PK>
 static int launch_fwd_buf(int D, const FwdK& k, hipStream_t s) {
   constexpr int W = fwd_waves(K, PK, ACT);
-  if (k.win) {
+  if (k.tps) {
     if (k.xb) {  // bf16 windows (sum / mean)
       if constexpr (PK == PK_SUM && W % 8 == 0)
         return k.ws_small ? launch_fwd<K, FWD_NPL, W / 2, ACT, false, true, PK, false, true, BT, true>(k, s)
@@ -1472,11 +1475,22 @@ static int fwd_run(const GlFwdArgs* a, void* ws, const FwdPlan& q, hipStream_t s
         window_staging(a->win, a->win_width, a->D, q.waves / 2, q.cpg, a->G, &k.ww, &k.npw, WS_SLOTS / 2, ib)) {
       k.win = a->win;
       k.ws_small = 1;
+      k.tps = WS_TILES;
     } else if (window_staging(a->win, a->win_width, a->D, q.waves, q.cpg, a->G, &k.ww, &k.npw, WS_SLOTS, ib)) {
       k.win = a->win;
+      k.tps = WS_TILES;
+    } else if (a->K == 8 && (a->pool == GL_POOL_MAX || a->pool == GL_POOL_TOPK_MEAN)) {
+      // max / top-k over at most 2048 inputs: a 64-KiB region holds 2 or more tiles, so one barrier
+      // (of 12 waves at 3 per SIMD) and one copy serve them all.  Forward at 2M neurons, 128 tokens,
+      // one tile per barrier -> staged: max D = 500 264 -> 227 us, D = 2000 326 -> 315, 10M neurons
+      // and 256 tokens at D = 1024 2.50 -> 2.15 ms; top-8 D = 1024 490 -> 454.  Not for sum / mean
+      // (two workgroups per CU hide the barrier: D = 1024 719 -> 776 us), nor at fan-in 16 (max 778
+      // -> 840 us), nor with one tile per region (top-8 at D = 4096 4.92 -> 5.23 ms).
+      const int tps = stage_tiles(a->D, 16, XTILE_DB, b_pad / BT);
+      if (tps >= 2) k.tps = tps, k.ww = a->D, k.npw = 1;
     }
     // fp32 X, sum / mean over full tiles of 4097..8192 inputs: two-token tiles (8-byte slots)
-    k.tb = !k.xb && pool_kind(a->pool) == PK_SUM && !k.win && tiles_of_two(a->D) ? 2 : BT;
+    k.tb = !k.xb && pool_kind(a->pool) == PK_SUM && !k.tps && tiles_of_two(a->D) ? 2 : BT;
     k.n_tiles = b_pad / k.tb;
     if (k.xb)
       GL_TRY(launch_tile_x_bf16x4(a->X, a->sxb, a->B, a->D, b0, k.n_tiles, xt, s));
