@@ -24,7 +24,7 @@ PROBE_SRC = CSRC / "probe" / "gl_lds_probe.hip"
 PROBE_LIB = OUT_DIR / "libgl_lds_probe.so"
 ARCH = "gfx950"
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
-SOURCES = ["gl_abi.hip", "gl_forward.hip", "gl_backward.hip", "gl_max_bwd.hip", "gl_edges.hip", "gl_adam.hip",
+SOURCES = ["gl_abi.hip", "gl_forward.hip", "gl_backward.hip", "gl_record.hip", "gl_max_bwd.hip", "gl_edges.hip", "gl_adam.hip",
            "gl_sched.hip", "gl_cover.hip"]
 FLAGS = [
     "-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}",

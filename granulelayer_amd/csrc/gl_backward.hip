@@ -1555,7 +1555,7 @@ static bool dense_dz(int pool, int act) {
   return is_smooth(pool) || (act == GL_ACT_GELU && (pool == GL_POOL_MEAN || pool == GL_POOL_SUM));
 }
 
-static BwdPlan bwd_plan(int B, int D, int G, int S, int K, bool smooth = false, size_t dz_budget = 0) {
+static BwdPlan bwd_plan(int B, int D, int G, int S, int K, bool smooth = false, size_t dz_budget = 0, bool rec = false) {
   BwdPlan q;
   q.bc_max = B < BWD_TOKEN_CHUNK ? B : BWD_TOKEN_CHUNK;
   if (smooth) {
@@ -1611,7 +1611,7 @@ static BwdPlan bwd_plan(int B, int D, int G, int S, int K, bool smooth = false, 
       q.UQs = ceil_div(q.U, 8 * q.QLs);
     }
   }
-  q.xt_bytes = (size_t)round_up((long long)q.tiles_max * D * 16, 256);
+  q.xt_bytes = (size_t)round_up((rec ? round_up(q.bc_max, 64) * 4 : (long long)q.tiles_max * 16) * D, 256);
   q.c1_bytes = (size_t)round_up((long long)G * q.cap_max * 4, 256);
   q.mask_bytes = (size_t)round_up((long long)G * S * q.rs_max * 4, 256);
   q.dz_bytes = smooth ? (size_t)round_up((long long)G * S * q.cap_max * 4, 256) : 0;
@@ -1814,12 +1814,17 @@ static bool dx_short_segments(const GlBwdArgs* a) {
   return (long long)a->S * a->K * FW < 64 * reach;
 }
 
+// the dW pass on the matrix cores (gl_record.hip), for neurons whose dz is a 0 / 1 mask times c1
+static bool bwd_rec_layer(const GlBwdArgs* a) {
+  return a->act != GL_ACT_GELU && record_layer(a->K, a->rec_shift, a->pool, a->w_dtype);
+}
+
 extern "C" int gl_bwd_workspace(const GlBwdArgs* a, size_t* bytes) {
   if (!a || !bytes) return GL_ERR_ARG;
   GL_TRY(check_layer(a->B, a->D, a->G, a->S, a->K, a->act, a->pool, a->X, a->idx, a->W, a->bias, a->counts,
                      a->x_dtype, a->w_dtype));
   const bool smooth = dense_dz(a->pool, a->act);
-  BwdPlan q = bwd_plan(a->B, a->D, a->G, a->S, a->K, smooth, a->dz_budget);
+  BwdPlan q = bwd_plan(a->B, a->D, a->G, a->S, a->K, smooth, a->dz_budget, bwd_rec_layer(a));
   GL_TRY(check_topk(a->pool, a->topk, a->S));
   GL_TRY(check_rec_shift(a->rec_shift, a->S, a->sched));
   GL_TRY(check_smooth(a->pool, a->pool_param, a->act));
@@ -1852,7 +1857,7 @@ extern "C" int gl_bwd(const GlBwdArgs* a, void* stream) {
   const bool smooth = dense_dz(a->pool, a->act);
   if (is_smooth(a->pool) && (!a->pre && !(a->pool == GL_POOL_LME && a->lse))) return GL_ERR_ARG;  // coefficients need pre
   if (a->pool == GL_POOL_SOFTMAX && !a->lse) return GL_ERR_ARG;
-  BwdPlan q = bwd_plan(a->B, a->D, a->G, a->S, a->K, smooth, a->dz_budget);
+  BwdPlan q = bwd_plan(a->B, a->D, a->G, a->S, a->K, smooth, a->dz_budget, bwd_rec_layer(a));
   const int sps = a->sps > 1 ? a->sps : 1, gs = a->sps > 1 ? a->gs : a->S;  // checked by gl_bwd_workspace
   char* ws = (char*)a->ws;
   float4* xt = (float4*)ws;
@@ -1889,7 +1894,10 @@ extern "C" int gl_bwd(const GlBwdArgs* a, void* stream) {
     // two-token fp32 tiles: half the gathers and tile overheads per token for one widening per value)
     const bool xb = (wide && a->x_dtype == GL_DTYPE_BF16) || (win && xbw);
     const int tb = wide && !xb ? 2 : BT;
-    if (xb)
+    const bool rec = bwd_rec_layer(a) && record_aligned(a->W, a->bias, a->idx) && ((uintptr_t)a->dW & 15) == 0;
+    if (rec)
+      GL_TRY(launch_slice_x(a->X, a->sxb, a->x_dtype, a->B, a->D, b0, ceil_div(Bc, 64), (float*)xt, s));
+    else if (xb)
       GL_TRY(launch_tile_x_bf16x4(a->X, a->sxb, a->B, a->D, b0, n_tiles, xt, s));
     else
       GL_TRY(launch_tile_x(a->X, a->sxb, a->x_dtype, a->B, a->D, b0, n_tiles * BT / tb, xt, s, tb));
@@ -1958,7 +1966,11 @@ extern "C" int gl_bwd(const GlBwdArgs* a, void* stream) {
       bk.fm_tiles = ceil_div(a->B, BT);
       bk.fm_t0 = b0 / BT;
     }
-    GL_TRY(launch_bwd_w_any(a->K, a->act, bk, s));
+    if (rec)
+      GL_TRY(launch_rec_bwd_w(a->act, (const float*)xt, a->idx, W, bias, a->counts, c1t, a->dW, a->db, mask, a->D, a->G,
+                              a->S, cap, Bc, T, s));
+    else
+      GL_TRY(launch_bwd_w_any(a->K, a->act, bk, s));
     DxK dk{(const uint32_t*)(eb + h.off_rec), (const uint32_t*)(eb + h.off_seg_ptr),
            (const int32_t*)(eb + h.off_seg_unit), (const uint32_t*)(eb + h.off_seg_begin), c1t, mask, W, part,
            NS, a->D, a->S, q.P, q.U, q.QL, q.UQ, q.FR, cap, cap / (64 * T), sps, gs};

@@ -1269,6 +1269,7 @@ struct FwdPlan {
   int npl, waves, cpg, bf, n_passes;
   long long n_chunks;
   size_t xt_bytes, part_bytes, slot_bytes;
+  bool rec;  // record kernels (gl_record.hip): chunks of REC_CHUNK slots, X in slices of 64 tokens
 };
 
 // bytes of partial results (values, plus slots for max / top-k) one token of a pass holds
@@ -1279,12 +1280,18 @@ static long long fwd_part_per_token(const GlFwdArgs* a, long long n_chunks) {
   return n_chunks * kp * 4 * (sel ? 2 : 1);
 }
 
+static bool fwd_rec(const GlFwdArgs* a) {
+  return record_layer(a->K, a->rec_shift, a->pool, a->w_dtype) && record_aligned(a->W, a->bias, a->idx);
+}
+
 // plan with token chunks of at most bf_cap tokens (<= 0: no cap beyond the part budget)
-static FwdPlan fwd_plan(const GlFwdArgs* a, long long bf_cap = 0) {
+// rec: with the record kernels (fwd_rec)
+static FwdPlan fwd_plan(const GlFwdArgs* a, bool rec, long long bf_cap = 0) {
   FwdPlan q;
+  q.rec = rec;
   q.npl = FWD_NPL;
   q.waves = fwd_waves(a->K, fwd_pool_kind(a), a->act);
-  q.cpg = ceil_div(a->S, 64 * q.npl);
+  q.cpg = ceil_div(a->S, q.rec ? REC_CHUNK : 64 * q.npl);
   q.n_chunks = (long long)a->G * q.cpg;
   const long long kp = a->pool == GL_POOL_TOPK_MEAN ? a->topk : (pool_smooth(a->pool) ? 3 : 1);
   const bool sel = a->pool == GL_POOL_MAX || a->pool == GL_POOL_TOPK_MEAN;
@@ -1295,9 +1302,10 @@ static FwdPlan fwd_plan(const GlFwdArgs* a, long long bf_cap = 0) {
   if (bf < BT) bf = BT;
   if (bf_cap > 0 && bf > bf_cap) bf = bf_cap;
   if (bf > b_all) bf = b_all;
+  if (q.rec && bf < b_all && bf >= 64) bf = bf / 64 * 64;  // whole slices
   q.bf = (int)bf;
   q.n_passes = ceil_div(a->B, q.bf);
-  q.xt_bytes = (size_t)round_up((long long)q.bf * a->D * 4, 256);
+  q.xt_bytes = (size_t)round_up((q.rec ? round_up(q.bf, 64) : (long long)q.bf) * a->D * 4, 256);
   q.part_bytes = (size_t)round_up(q.n_chunks * q.bf * kp * 4, 256);
   q.slot_bytes = sel ? q.part_bytes : 0;  // candidate slots
   return q;
@@ -1453,6 +1461,15 @@ static int fwd_run(const GlFwdArgs* a, void* ws, const FwdPlan& q, hipStream_t s
     const int b_pad = (int)round_up(Bc, BT);
     float* pre = a->pre + (long long)b0 * a->G;
     int32_t* winner = a->winner ? a->winner + (long long)b0 * a->G * kpe : nullptr;
+    if (q.rec) {
+      GL_TRY(launch_slice_x(a->X, a->sxb, a->x_dtype, a->B, a->D, b0, ceil_div(b_pad, 64), (float*)xt, s));
+      GL_TRY(launch_rec_fwd(a->act, (const float*)xt, a->idx, (const float*)a->W, (const float*)a->bias, a->counts, part,
+                            q.n_chunks, a->D, a->S, q.cpg, b_pad, s));
+      GL_LAUNCH(GL_KERNEL_FWD_FINALIZE, fwd_finalize_kernel, dim3((unsigned)ceil_div(a->G, 32), (unsigned)ceil_div(b_pad, 32)),
+                dim3(256), 0, s, part, a->counts, pre, Bc, a->G, q.cpg, b_pad, 0, a->pool);
+      GL_CHECK_LAUNCH();
+      continue;
+    }
     FwdK k{xt, a->idx, (const float*)a->W, (const float*)a->bias, a->counts, part, pslot, kpe, a->sched, nullptr, q.n_chunks, a->D, a->S, q.cpg,
            b_pad / BT, b_pad, ceil_div(a->S, SCHED_WIN), a->G, 0, 0, a->rec_shift,
            smooth_scale(a->pool, a->pool_param), a->pool_param, smooth_pint(a->pool, a->pool_param)};
@@ -1591,8 +1608,15 @@ static int scratch_address(int* dev_out, void** out) {
 }
 
 // the largest token chunk whose tiles and partials fit the scratch (0: not even one tile)
-static long long static_chunk(const GlFwdArgs* a) {
-  const long long cpg = ceil_div(a->S, 64 * FWD_NPL);
+static long long static_chunk(const GlFwdArgs* a, bool rec) {
+  const long long cpg = ceil_div(a->S, rec ? REC_CHUNK : 64 * FWD_NPL);
+  if (rec) {  // X in whole slices of 64 tokens
+    const long long part = fwd_part_per_token(a, (long long)a->G * cpg), xs = (long long)a->D * 256;
+    const long long room = (long long)GL_FWD_STATIC_SCRATCH_BYTES - 3 * 256;
+    const long long slices = room / (xs + 64 * part);
+    if (slices > 0) return slices * 64;
+    return room > xs ? (room - xs) / part / BT * BT : 0;
+  }
   const long long per_token = fwd_part_per_token(a, (long long)a->G * cpg) + (long long)a->D * 4;
   const long long room = (long long)GL_FWD_STATIC_SCRATCH_BYTES - 3 * 256;  // three sections rounded to 256
   return room / per_token / BT * BT;
@@ -1612,8 +1636,12 @@ extern "C" int gl_fwd_workspace(const GlFwdArgs* a, size_t* bytes) {
   int32_t sps = a->sps, gs = a->gs;
   GL_TRY(check_geometry(a->G, a->S, &sps, &gs));
   if (sps > 1 && a->rec_shift > 0) return GL_ERR_UNSUPPORTED;
-  FwdPlan q = fwd_plan(a);
+  FwdPlan q = fwd_plan(a, false);
   *bytes = q.xt_bytes + q.part_bytes + q.slot_bytes;
+  if (record_layer(a->K, a->rec_shift, a->pool, a->w_dtype)) {  // room for either path, whatever the pointers
+    q = fwd_plan(a, true);
+    if (*bytes < q.xt_bytes + q.part_bytes) *bytes = q.xt_bytes + q.part_bytes;
+  }
   return 0;
 }
 
@@ -1632,7 +1660,7 @@ extern "C" int gl_fwd(const GlFwdArgs* a, void* stream) {
   GL_TRY(gl_fwd_workspace(a, &need));
   if (!a->ws || a->ws_bytes < need) return GL_ERR_WORKSPACE;
   if (a->sched && a->K != 8) return GL_ERR_UNSUPPORTED;
-  return fwd_run(a, a->ws, fwd_plan(a), (hipStream_t)stream);
+  return fwd_run(a, a->ws, fwd_plan(a, fwd_rec(a)), (hipStream_t)stream);
 }
 
 extern "C" int gl_fwd_static(const GlFwdArgs* a, void* stream) {
@@ -1641,9 +1669,12 @@ extern "C" int gl_fwd_static(const GlFwdArgs* a, void* stream) {
   size_t need = 0;
   GL_TRY(gl_fwd_workspace(a, &need));  // argument checks; ws / ws_bytes are ignored
   if (a->sched && a->K != 8) return GL_ERR_UNSUPPORTED;
-  const long long bf = static_chunk(a);
+  // a record layer whose 128-slot partials do not fit runs the per-neuron kernels (256-slot partials)
+  bool rec = fwd_rec(a);
+  long long bf = static_chunk(a, rec);
+  if (rec && bf < BT) rec = false, bf = static_chunk(a, false);
   if (bf < BT) return GL_ERR_SCRATCH;
-  const FwdPlan q = fwd_plan(a, bf);
+  const FwdPlan q = fwd_plan(a, rec, bf);
   if (q.xt_bytes + q.part_bytes + q.slot_bytes > (size_t)GL_FWD_STATIC_SCRATCH_BYTES) return GL_ERR_SCRATCH;
   // Calls on one GPU share its scratch.  A call waits on the device's "last use" event before its
   // launches and records it after them, so calls on different streams of one GPU run one after

@@ -86,6 +86,24 @@ struct MaxEvKArgs {
 };
 int launch_max_events(int K, int act, const MaxEvKArgs& a, hipStream_t s);
 
+// Layers with one fan-in-16 record per 16 slots (gl_record.hip): sum / mean forward and dW pass as dense
+// 16 x 16 products on the matrix cores.  X goes through slices of 64 tokens ([slice][D][64] fp32), a
+// wave takes REC_CHUNK slots.  record_layer: the layer qualifies (workspaces are sized by it alone,
+// whatever the pointers); record_aligned: these pointers do too.  Other layers with shared records
+// (other shifts, fan-in 8, bf16 parameters, views off a 16-byte boundary) run the per-neuron kernels.
+constexpr int REC_CHUNK = 128;
+bool record_layer(int K, int rec_shift, int pool, int w_dtype);
+inline bool record_aligned(const void* a, const void* b, const void* c) {
+  return (((uintptr_t)a | (uintptr_t)b | (uintptr_t)c) & 15) == 0;
+}
+int launch_slice_x(const void* X, long long sxb, int x_dtype, int B, int D, int b0, int n_slices, float* xs,
+                   hipStream_t s);
+int launch_rec_fwd(int act, const float* xs, const int32_t* idx, const float* W, const float* bias, const int32_t* counts,
+                   float* part, long long n_chunks, int D, int S, int cpg, int b_pad, hipStream_t s);
+int launch_rec_bwd_w(int act, const float* xs, const int32_t* idx, const float* W, const float* bias,
+                     const int32_t* counts, const float* c1t, float* dW, float* db, uint32_t* mask, int D, int G, int S,
+                     int cap, int Bc, int T, hipStream_t s);
+
 // Launch trace (gl_trace_begin): record an event pair around one kernel launch.
 void trace_before(hipStream_t s, int kernel_id);
 void trace_after(hipStream_t s);

@@ -206,3 +206,94 @@ def test_cover_topk16_at_the_c5_shape():
     (mW, mb, mX), (uW, ub, uX) = bnd["mag"], bnd["unc"]
     assert_parity(xd.grad.cpu().numpy(), dX, mX, uX, what="C5 Cover-TopK/16 dX")
     assert_parity(lay.weight.main_grad.view(-1, 16, 16)[rows].cpu().numpy().reshape(-1, 16), dW, mW, uW, what="dW")
+
+
+# ---- the record kernels (gl_record.hip) ------------------------------------------------------------
+# (D, neurons per pool, pools, B, x dtype): one token, the edges of the 64-token slices and of the dX
+# slabs (64 / 128 / 256), pools of one partial record, of a partial chunk of 8 records, of chunks and a bit
+RECORD_CASES = [
+    (64, 5, 3, 1, torch.float32),
+    (100, 16, 7, 63, torch.float32),
+    (96, 130, 5, 64, torch.bfloat16),
+    (33, 117, 4, 65, torch.float32),
+    (512, 300, 3, 129, torch.float32),
+    (40, 1040, 2, 260, torch.bfloat16),
+    (64, 40, 3, 1030, torch.float32),
+]
+
+
+def _record_layer(D, per, G, seed=0):
+    """A compact layer with random records (padded neurons' weights and biases are not zero: only the
+    kernels' own masks keep them out)."""
+    S = -(-per // 16) * 16
+    lay = CoverTopK16Layer(D, G * per, G, S, pooling="mean", device=DEV)
+    gen = torch.Generator().manual_seed(seed)
+    rec = torch.stack([torch.randperm(D, generator=gen)[:16].sort().values for _ in range(G * S // 16)])
+    with torch.no_grad():
+        lay.indices.copy_(rec.to(torch.int32).view(lay.indices.shape))
+        lay.weight.copy_(torch.randn(lay.weight.shape, generator=gen) / 4)
+        lay.bias.copy_(torch.randn(lay.bias.shape, generator=gen) / 4)
+    return lay
+
+
+@pytest.mark.parametrize("act,pool", [("relu", "sum"), ("identity", "mean"), ("gelu", "sum")])
+@pytest.mark.parametrize("case", RECORD_CASES, ids=lambda c: f"D{c[0]}n{c[1]}B{c[3]}{str(c[4])[6:]}")
+def test_record_kernels_match_oracle(case, act, pool):
+    from granulelayer_amd import LevelSpec, PhysicalPlan
+    from granulelayer_amd.autograd import Level1Runtime
+
+    D, per, G, B, xdt = case
+    lay = _record_layer(D, per, G)
+    L = lay.layout
+    S = L.slots_per_group
+    gen = torch.Generator().manual_seed(B)
+    x, dy = torch.randn(B, D, generator=gen).to(xdt), torch.randn(B, G, generator=gen)
+    counts = L.counts_tensor("cpu").numpy()
+    idx = lay.indices.cpu().numpy().reshape(-1, 16).repeat(16, 0)
+    w, b = lay.weight.detach().cpu().numpy().reshape(-1, 16), lay.bias.detach().cpu().numpy().reshape(-1)
+    xn = x.float().numpy()
+    want, mag = O.forward(xn, idx, w, b, counts, S, act, pool, with_mag=True)
+    rt = Level1Runtime(L, lay.indices, LevelSpec(pool, activation=act), PhysicalPlan())
+    xd = x.to(DEV)
+    got = rt.forward(xd, lay.weight, lay.bias)
+    assert_parity(got["pre"].cpu().numpy(), want, mag, what="pre")
+    dw, db = torch.zeros(L.weight_shape, device=DEV), torch.zeros(L.bias_shape, device=DEV)
+    dx = rt.backward(xd, lay.weight, lay.bias, dy.to(DEV), {"pre": got["pre"]}, "minimal_stats", dw, db)
+    dW, dB, dX, bnd = O.backward(xn, idx, w, b, counts, S, dy.numpy(), act, pool, with_bounds=True)
+    (mW, mb, mX), (uW, ub, uX) = bnd["mag"], bnd["unc"]
+    assert_parity(dw.cpu().numpy().reshape(-1, 16), dW, mW, uW, what="dW")
+    assert_parity(db.cpu().numpy().reshape(-1), dB, mb, ub, what="db")
+    assert_parity(dx.cpu().numpy(), dX, mX, uX, what="dX")
+    valid = L.valid_mask("cpu").reshape(-1).numpy()
+    assert not dw.cpu().numpy().reshape(-1, 16)[~valid].any() and not db.cpu().numpy().reshape(-1)[~valid].any()
+    # views off a 16-byte boundary run the per-neuron kernels: the same sums in another order
+    off = torch.empty(lay.weight.numel() + 1, device=DEV)[1:].view(lay.weight.shape).copy_(lay.weight.detach())
+    pre = rt.forward(xd, off, lay.bias)["pre"].cpu().numpy()
+    assert_parity(pre, want, mag, what="pre (unaligned weights)")
+
+
+def test_record_forward_in_token_passes_and_without_a_workspace():
+    """A part budget of 20 tokens' partials, whole batches and gl_fwd_static give the same bits: a
+    token's sums do not depend on the tokens beside it."""
+    import ctypes
+
+    from granulelayer_amd import LevelSpec, PhysicalPlan
+    from granulelayer_amd import _native as N
+    from granulelayer_amd.autograd import Level1Runtime
+    from granulelayer_amd.backend import _ptr, _stream
+
+    lay = _record_layer(128, 520, 50)
+    L = lay.layout
+    x = torch.randn(150, 128, device=DEV)
+    chunks = L.groups * -(-L.slots_per_group // 128)
+    outs = []
+    for budget in (None, chunks * 4 * 20, chunks * 4 * 100):
+        rt = Level1Runtime(L, lay.indices, LevelSpec("sum", activation="relu"), PhysicalPlan(), None, budget)
+        outs.append(rt.forward(x, lay.weight, lay.bias)["pre"])
+    pre = torch.empty_like(outs[0])
+    a = N.GlFwdArgs(X=_ptr(x), sxb=128, x_dtype=N.GL_DTYPE_F32, B=150, D=128, G=L.groups, S=L.slots_per_group, K=16,
+                    act=N.GL_ACT["relu"], pool=N.GL_POOL["sum"], rec_shift=4, idx=_ptr(lay.indices), W=_ptr(lay.weight),
+                    bias=_ptr(lay.bias), counts=_ptr(rt.counts_i32), pre=_ptr(pre))
+    assert N.library().lib.gl_fwd_static(ctypes.byref(a), ctypes.c_void_p(_stream(x.device))) == 0
+    for o in (*outs[1:], pre):
+        assert torch.equal(o, outs[0])
