@@ -10,11 +10,11 @@
 // row (a slice of 4096 inputs is 1 MiB, so the slices in use stay in an XCD's L2), and a wave loads
 // the 16 rows of a record with four 1-KiB loads straight into MFMA operands, with no LDS.
 //
-// Bounds: at 12.6M neurons, 512 tokens, 4096 inputs the forward runs 2.08 ms and the dW pass 4.69 ms
+// Bounds: at 12.6M neurons, 512 tokens, 4096 inputs the forward runs 2.17 ms and the dW pass 4.85 ms
 // (7.47 and 10.5 in the per-neuron kernels; the products alone take 1.31 and 2.62 ms at the 157 TFLOP/s
 // of fp32 MFMA).  Beside the MFMAs the forward issues 32 VALU per record and slice (the activation and
 // the sum), the dW pass ~110 (dz, mask bits, db).  The second layout of X that dW needs (inputs, not
-// tokens, across lanes) read again from memory ran 5.70 ms: 16-byte pieces of 64 rows per load, and
+// tokens, across lanes) read again from memory ran 5.70 ms (4.69 then): 16-byte pieces of 64 rows per load, and
 // the rows no longer in the 32-KiB L1.  Loads, not LDS, feed the products because a slice of 64
 // tokens of a wide layer (1 MiB) fits no LDS, while 4 tokens (what does fit) leave 3/4 of a tile idle.
 //
@@ -67,8 +67,28 @@ __device__ __forceinline__ float rows_sum(float c) {
   return __uint_as_float(p32[0]) + __uint_as_float(p32[1]);
 }
 
-// the chunk of a wave: pool g, first slot, valid records, and per record the lane's 4 weights
-// (neuron m, k = 4 G + j), the byte offsets of its 4 input rows (inputs 4 G + j, tokens 4 m ..)
+// Product j of a record takes its edges 4 j + G (k-slot G).  The MFMA adds its 4 k-slots in order,
+// each as an fma, so z is the fma chain over k = 0 .. 15 from the bias that the per-neuron kernels
+// run, bit for bit: the ReLU decisions are the same (edges 4 G + j, which one 16-byte load per lane
+// would give, differ from it in rounding and so in the sign of a few z near 0).  The edges are loaded
+// 4 per lane (k = 4 G ..) and exchanged: rec_transpose turns component j of lane (m, G) into component
+// G of lane (m, j), a 4 x 4 transpose over the wave's four rows of 16 lanes.
+__device__ __forceinline__ uint4 rec_transpose(uint4 v) {
+  const auto a = __builtin_amdgcn_permlane32_swap(v.x, v.z, false, false);
+  const auto b = __builtin_amdgcn_permlane32_swap(v.y, v.w, false, false);
+  const auto c = __builtin_amdgcn_permlane16_swap(a[0], b[0], false, false);
+  const auto d = __builtin_amdgcn_permlane16_swap(a[1], b[1], false, false);
+  return make_uint4(c[0], c[1], d[0], d[1]);
+}
+// the lane's weights of neuron m (w: its row + 4 G), zero for a padded slot
+__device__ __forceinline__ float4 rec_weights(const float* w, bool valid) {
+  uint4 v = *reinterpret_cast<const uint4*>(w);
+  if (!valid) v = make_uint4(0u, 0u, 0u, 0u);
+  v = rec_transpose(v);
+  return make_float4(__uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z), __uint_as_float(v.w));
+}
+
+// the chunk of a wave: pool g, first slot, valid slots and records
 struct RecChunk {
   long long rec0;  // first record (global)
   int g, s_lo, n_g, nrec;
@@ -120,12 +140,11 @@ __global__ void __launch_bounds__(REC_WAVES * 64, 2) rec_fwd_kernel(RecFwdK p) {
   for (int r = 0; r < REC_PER_WAVE; ++r) {
     const long long rec = c.rec0 + (r < c.nrec ? r : 0);  // in bounds; records past the pool are skipped
     const int left = c.n_g - c.s_lo - r * REC_N;          // valid neurons of the record
-    w[r] = *reinterpret_cast<const float4*>(p.W + (rec * REC_N + m) * 16 + 4 * G);
-    if (m >= left) w[r] = make_float4(0.f, 0.f, 0.f, 0.f);
+    w[r] = rec_weights(p.W + (rec * REC_N + m) * 16 + 4 * G, m < left);
     bias[r] = *reinterpret_cast<const float4*>(p.bias + rec * REC_N + 4 * G);
-    const int4 d = *reinterpret_cast<const int4*>(p.idx + rec * 16 + 4 * G);
-    off[r][0] = row_off(d.x, p.D) + m * 16u, off[r][1] = row_off(d.y, p.D) + m * 16u;
-    off[r][2] = row_off(d.z, p.D) + m * 16u, off[r][3] = row_off(d.w, p.D) + m * 16u;
+    const uint4 d = rec_transpose(*reinterpret_cast<const uint4*>(p.idx + rec * 16 + 4 * G));
+    off[r][0] = row_off((int)d.x, p.D) + m * 16u, off[r][1] = row_off((int)d.y, p.D) + m * 16u;
+    off[r][2] = row_off((int)d.z, p.D) + m * 16u, off[r][3] = row_off((int)d.w, p.D) + m * 16u;
   }
   const int last = c.n_g - c.s_lo - (c.nrec - 1) * REC_N;  // valid neurons of the chunk's last record
   float* out = p.part + chunk * p.b_pad + 4 * m;
@@ -204,12 +223,11 @@ __global__ void __launch_bounds__(REC_WAVES * 64, 2) rec_bwd_w_kernel(RecBwdK p)
   for (int r = 0; r < REC_PER_WAVE; ++r) {
     const long long rec = c.rec0 + (r < c.nrec ? r : 0);
     const int left = c.n_g - c.s_lo - r * REC_N;
-    w[r] = *reinterpret_cast<const float4*>(p.W + (rec * REC_N + m) * 16 + 4 * G);
-    if (m >= left) w[r] = make_float4(0.f, 0.f, 0.f, 0.f);
+    w[r] = rec_weights(p.W + (rec * REC_N + m) * 16 + 4 * G, m < left);
     bias[r] = m < left ? p.bias[rec * REC_N + m] : 0.f;
-    const int4 d = *reinterpret_cast<const int4*>(p.idx + rec * 16 + 4 * G);
-    off[r][0] = row_off(d.x, p.D) + m * 16u, off[r][1] = row_off(d.y, p.D) + m * 16u;
-    off[r][2] = row_off(d.z, p.D) + m * 16u, off[r][3] = row_off(d.w, p.D) + m * 16u;
+    const uint4 d = rec_transpose(*reinterpret_cast<const uint4*>(p.idx + rec * 16 + 4 * G));
+    off[r][0] = row_off((int)d.x, p.D) + m * 16u, off[r][1] = row_off((int)d.y, p.D) + m * 16u;
+    off[r][2] = row_off((int)d.z, p.D) + m * 16u, off[r][3] = row_off((int)d.w, p.D) + m * 16u;
     dw[r] = v4f{0.f, 0.f, 0.f, 0.f};
     dbv[r] = 0.f;
   }
@@ -227,7 +245,7 @@ __global__ void __launch_bounds__(REC_WAVES * 64, 2) rec_bwd_w_kernel(RecBwdK p)
       constexpr int r = decltype(rc)::value;
       if (r >= c.nrec) return;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) *reinterpret_cast<float4*>(&xl[(4 * G + j) * REC_XROW + 4 * m]) = xc[j];
+      for (int j = 0; j < 4; ++j) *reinterpret_cast<float4*>(&xl[(4 * j + G) * REC_XROW + 4 * m]) = xc[j];
       if constexpr (r + 1 < REC_PER_WAVE) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) xn[j] = ld_row(xr, off[r + 1][j]);

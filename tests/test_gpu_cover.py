@@ -266,10 +266,23 @@ def test_record_kernels_match_oracle(case, act, pool):
     assert_parity(dx.cpu().numpy(), dX, mX, uX, what="dX")
     valid = L.valid_mask("cpu").reshape(-1).numpy()
     assert not dw.cpu().numpy().reshape(-1, 16)[~valid].any() and not db.cpu().numpy().reshape(-1)[~valid].any()
-    # views off a 16-byte boundary run the per-neuron kernels: the same sums in another order
+    # views off a 16-byte boundary run the per-neuron kernels: the same z bit for bit (pools of one
+    # slot show them), the same sums in another order
     off = torch.empty(lay.weight.numel() + 1, device=DEV)[1:].view(lay.weight.shape).copy_(lay.weight.detach())
     pre = rt.forward(xd, off, lay.bias)["pre"].cpu().numpy()
     assert_parity(pre, want, mag, what="pre (unaligned weights)")
+
+
+def test_record_z_has_the_bits_of_the_per_neuron_kernels():
+    from granulelayer_amd import LevelSpec, PhysicalPlan
+    from granulelayer_amd.autograd import Level1Runtime
+
+    lay = _record_layer(200, 1, 700)
+    rt = Level1Runtime(lay.layout, lay.indices, LevelSpec("sum", activation="identity"), PhysicalPlan())
+    x = torch.randn(70, 200, device=DEV)
+    w = lay.weight.detach()
+    off = torch.empty(w.numel() + 1, device=DEV)[1:].view(w.shape).copy_(w)  # not 16-byte aligned: per-neuron kernels
+    assert torch.equal(rt.forward(x, w, lay.bias)["pre"], rt.forward(x, off, lay.bias)["pre"])
 
 
 def test_record_forward_in_token_passes_and_without_a_workspace():
