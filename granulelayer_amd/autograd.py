@@ -92,6 +92,11 @@ def dact_torch(x: torch.Tensor, name: str) -> torch.Tensor:
     raise NotImplementedError(f"out-activation {name!r}")
 
 
+def _g_pre(dy: torch.Tensor, pre: torch.Tensor, name: str) -> torch.Tensor:
+    """dL/dpre = dy * act'(pre); an identity out-activation's factor of 1 needs no launches."""
+    return dy.float() if name == "identity" else dy.float() * dact_torch(pre, name)
+
+
 @dataclass
 class Units:
     """Level-1 pooling units (kernels/ops.py:30-56): one unit per group for a single level."""
@@ -267,7 +272,7 @@ def _level1_backward(rt: Level1Runtime, xc, wc, bc, dy, saved: Dict[str, torch.T
     if "pre" not in saved or (need is not None and need not in saved):
         saved.update(rt.forward(xc, wc, bc, track_ids=True))
         recomputed = True
-    g_pre = dy.float() * dact_torch(saved["pre"], lv.out_activation)
+    g_pre = _g_pre(dy, saved["pre"], lv.out_activation)
     return rt.backward(xc, wc, bc, g_pre.contiguous(), saved, policy, dw_buf, db_buf, recomputed)
 
 
@@ -282,7 +287,7 @@ def _chunked_selection_backward(rt: Level1Runtime, xc, wc, bc, dy, pre, policy, 
         xs = xc[s0:s0 + bc_tok]
         st = rt.forward(xs, wc, bc, track_ids=True)
         p = st["pre"] if pre is None else pre[s0:s0 + bc_tok]
-        g = (dy[s0:s0 + bc_tok].float() * dact_torch(p, rt.level.out_activation)).contiguous()
+        g = _g_pre(dy[s0:s0 + bc_tok], p, rt.level.out_activation).contiguous()
         dx[s0:s0 + bc_tok] = rt.backward(xs, wc, bc, g, st, policy, dw_buf, db_buf, True)
         del st
     rt.last_info["backward_token_chunks"] = -(-B // bc_tok)

@@ -16,6 +16,7 @@ pointers.  Any refusal of the native library raises ``NativeError``; there is no
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import threading
 from typing import Dict, Optional
@@ -42,6 +43,15 @@ def _ptr(t: Optional[torch.Tensor]) -> int:
 
 def _stream(dev) -> int:
     return torch.cuda.current_stream(dev).cuda_stream
+
+
+_NO_SWITCH = contextlib.nullcontext()
+
+
+def _on(dev):
+    """``torch.cuda.device(dev)``, or nothing when dev is the current device already (the switch and
+    its return cost the smallest calls several microseconds)."""
+    return _NO_SWITCH if dev.index == torch.cuda.current_device() else torch.cuda.device(dev)
 
 
 def _x_operand(x: torch.Tensor):
@@ -194,7 +204,7 @@ class HipBackend:
                         sched=_ptr(self.schedule(rt)), win=_ptr(win_lo), win_width=win_width, pre=_ptr(pre),
                         winner=_ptr(winner), pool_param=self.pool_param(rt), lse=_ptr(lse),
                         part_budget=self.part_budget(rt), w_dtype=wcode)
-        with torch.cuda.device(x.device):
+        with _on(x.device):
             if relu_mask:
                 mb = self.lib.size_query("gl_fwd_mask_bytes", a)
                 if 0 < mb <= RELU_MASK_BUDGET:
@@ -237,19 +247,20 @@ class HipBackend:
         """Gather schedule of rt's index tensor for the forward / dW kernels (fan-in 8, one index
         record per slot), built on the GPU once per index tensor (gl_sched_build, the host
         builder's algorithm) and cached on rt; None otherwise."""
-        L, _, _, K = self._layer(rt)
-        G, S, sps, gs, counts = self._pools(rt)
+        L = rt.layout
+        K = L.fan_in
         if K != 8 or self.rec_shift(rt):
             return None
         key = (rt.idx.data_ptr(), rt.idx._version)
         cached = getattr(rt, "_hip_sched", None)
         if cached is not None and cached[0] == key:
             return cached[1]
+        G, S, sps, gs, counts = self._pools(rt)
         dev = rt.idx.device
         n = ctypes.c_size_t(0)
         self.lib.call("gl_sched_size", G, S, K, ctypes.byref(n))
         sched = torch.empty(n.value // 4, dtype=torch.int32, device=dev)
-        with torch.cuda.device(dev):
+        with _on(dev):
             self.lib.call("gl_sched_build", _ptr(rt.idx), _ptr(counts), L.input_dim, G, S, sps, gs, K, _ptr(sched),
                           ctypes.c_void_p(_stream(dev)))
         rt._hip_sched = (key, sched)
@@ -262,16 +273,16 @@ class HipBackend:
         when ``window_staging`` is off.  The library stages only the windows when they are narrow."""
         if not self.window_staging:
             return None, 0
-        L, _, _, K = self._layer(rt)
-        G, S, sps, gs, counts = self._pools(rt)
         key = (rt.idx.data_ptr(), rt.idx._version)
         cached = getattr(rt, "_hip_win", None)
         if cached is not None and cached[0] == key:
             return cached[1]
+        L, _, _, K = self._layer(rt)
+        G, S, sps, gs, counts = self._pools(rt)
         dev = rt.idx.device
         lo = torch.empty(G, dtype=torch.int32, device=dev)
         width = torch.empty(1, dtype=torch.int32, device=dev)
-        with torch.cuda.device(dev):
+        with _on(dev):
             self.lib.call("gl_window_build", _ptr(rt.idx), _ptr(counts), L.input_dim, G, S, sps, gs, K,
                           self.rec_shift(rt), _ptr(lo), _ptr(width), ctypes.c_void_p(_stream(dev)))
         out = (lo, int(width.item()))  # the launch needs the width on the host: one 4-byte copy
@@ -290,7 +301,7 @@ class HipBackend:
         a = N.GlEdgeArgs(idx=_ptr(rt.idx), counts=_ptr(counts), D=L.input_dim, G=G, S=S, K=K,
                          rec_shift=self.rec_shift(rt), sps=sps, gs=gs)
         dev = rt.idx.device
-        with torch.cuda.device(dev):
+        with _on(dev):
             eb, wb = self.lib.edges_size(a)
             edges = torch.empty(eb, device=dev, dtype=torch.uint8)
             ws = torch.empty(max(wb, 1), device=dev, dtype=torch.uint8)
@@ -357,7 +368,7 @@ class HipBackend:
                 raise ValueError("relu_mask does not come from this layer's forward of this batch")
             a.relu_mask = _ptr(rm)
         rt.last_info["backward_relu_mask"] = rm is not None
-        with torch.cuda.device(x.device):
+        with _on(x.device):
             need = self.lib.size_query("gl_bwd_workspace", a)
             ws = torch.empty(max(need, 1), device=x.device, dtype=torch.uint8)
             a.ws, a.ws_bytes = _ptr(ws), need
@@ -389,7 +400,7 @@ class HipBackend:
                          p_dtype=N.GL_DTYPE_BF16 if bf else N.GL_DTYPE_F32,
                          stochastic=int(bf and master is None and stochastic), master=_ptr(master),
                          seed=int(seed) & (2**64 - 1))
-        with torch.cuda.device(p.device):
+        with _on(p.device):
             self.lib.call("gl_adam", ctypes.byref(a), ctypes.c_void_p(_stream(p.device)))
 
 

@@ -33,6 +33,7 @@ import hashlib
 import math
 import time
 from dataclasses import dataclass
+from functools import cached_property
 from pathlib import Path
 from typing import Optional, Union
 
@@ -124,11 +125,11 @@ class CompactLayout:
     rec_shift: int = 4
     shared_indices: bool = True
 
-    @property
+    @cached_property
     def rows_per_group(self) -> int:
         return self.slots_per_group // 16
 
-    @property
+    @cached_property
     def blocks_per_group(self) -> int:
         return self.rows_per_group
 
@@ -140,15 +141,15 @@ class CompactLayout:
         s = torch.arange(self.slots_per_group, device=device)
         return (s[None, :] < self.counts_tensor(device)[:, None]).view(self.groups, self.rows_per_group, 16)
 
-    @property
+    @cached_property
     def index_shape(self):
         return (self.groups, self.rows_per_group, FAN_IN)
 
-    @property
+    @cached_property
     def weight_shape(self):
         return (self.groups, self.rows_per_group, 16, FAN_IN)
 
-    @property
+    @cached_property
     def bias_shape(self):
         return (self.groups, self.rows_per_group, 16)
 

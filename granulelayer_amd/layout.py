@@ -21,6 +21,7 @@ from __future__ import annotations
 import dataclasses
 import math
 from dataclasses import dataclass
+from functools import cached_property
 
 import torch
 
@@ -50,24 +51,24 @@ class SparseLayout:
             raise NotImplementedError("fragment-packed (Mode B, mma) storage is not on the MI355X path")
 
     # ---- partition -------------------------------------------------------
-    @property
+    @cached_property
     def base(self) -> int:
         return self.hidden_dim // self.groups
 
-    @property
+    @cached_property
     def rem(self) -> int:
         return self.hidden_dim % self.groups
 
-    @property
+    @cached_property
     def max_group(self) -> int:
         return self.base + (1 if self.rem else 0)
 
-    @property
+    @cached_property
     def blocks_per_group(self) -> int:
         nb = -(-self.max_group // self.block)
         return (nb + 3) // 4 * 4
 
-    @property
+    @cached_property
     def slots_per_group(self) -> int:
         return self.blocks_per_group * self.block
 
@@ -97,16 +98,16 @@ class SparseLayout:
         return s[None, :] < self.counts_tensor(device)[:, None]
 
     # ---- shapes ----------------------------------------------------------
-    @property
+    @cached_property
     def index_shape(self):
         G, NB, C, K = self.groups, self.blocks_per_group, self.block, self.fan_in
         return (G, NB, K) if self.shared_indices else (G, NB, C, K)
 
-    @property
+    @cached_property
     def weight_shape(self):
         return (self.groups, self.blocks_per_group, self.block, self.fan_in)
 
-    @property
+    @cached_property
     def bias_shape(self):
         return (self.groups, self.blocks_per_group, self.block)
 
