@@ -527,6 +527,7 @@ struct DxK {
   int D, S, P, U, QL, UQ, FR, cap, n_tc;
   int sps, gs;  // pool geometry (pool_base)
   int wbf;      // W stored as bf16: the edge's weight is the half of the 32-bit word at (offset / 2) & ~3
+  int Bc;       // dx_dense_kernel: tokens of the chunk
   int ql0;      // dx_dense_kernel: the pass's first unit range per XCD (its ranges are ql0 .. ql0 + QL - 1)
 };
 
@@ -1375,13 +1376,36 @@ __global__ void __launch_bounds__(WAVES * 64) bwd_smooth_kernel(BsK p) {
   }
 }
 
+// acc[f] += r, f wave-uniform: one uniform branch per feature, so every accumulator stays in its
+// registers (the asm comment tells the branches apart: merged into one with a computed index, the
+// accumulators went to scratch memory)
+template <int X, int T>
+__device__ __forceinline__ void dx_add_run(int f, const float (&r)[T], float (&acc)[FW][T]) {
+  if (f == X) {
+#pragma unroll
+    for (int j = 0; j < T; ++j) acc[X][j] += r[j];
+    asm volatile("; feature %0" ::"n"(X));
+  } else if constexpr (X + 1 < FW) {
+    dx_add_run<X + 1, T>(f, r, acc);
+  }
+}
+
 // dX of a smooth pool: dX[b, d] = sum over edges (n, k) -> d of dz[b, n] W[n, k], walking the
 // input-major edges like dx_kernel (one wave per feature range, unit range and token slice); per
 // edge every lane reads its T tokens of the neuron's dz row (T = 1, 2 or 4 for token chunks of up
 // to 64, 128 or 256 tokens; test_gpu_smooth's B = 130 case runs T = 4).  A segment's edges are sorted
 // by feature, so consecutive edges into one feature are summed in registers (a run) and the run is
-// added to that feature's sums in LDS when the feature changes: one uniform branch per run where
-// selecting one of FW register accumulators per edge cost FW * T multiply-adds and selects.
+// added to that feature's sums when the feature changes.
+//
+// Each edge's row offset, weight and feature are computed once, in the edge's own lane, and taken
+// with v_readlane: the row is one buffer load with the unit's resource and the offset as its scalar
+// offset, and a bit mask of the run starts replaces the comparison of features.  Built from scalars
+// per edge, the 64-bit row address, the resource and the comparisons took ~34 scalar instructions, and
+// their issue (one per 4 clocks and SIMD: 136 clocks per edge) bounded the kernel at T = 1 and 2.
+// Lanes past the chunk's Bc tokens load nothing (their offset is out of the resource's range).
+// LogMeanExp dX before -> now: 4M neurons, 64 tokens, 1024 inputs 1.82 -> 0.88 ms; 0.78M at fan-in 16,
+// 77 tokens, 1000 inputs 731 -> 535 us; 2M, 200 tokens, 8000 inputs 3.00 -> 1.96 ms; 12.6M, 256
+// tokens, 4096 inputs 11.3 -> 10.6 ms (there the 103 GB of row reads bound it: 9.8 TB/s).
 template <int K, int T>
 __global__ void __launch_bounds__(64) dx_dense_kernel(DxK p, const float* __restrict__ dz) {
   const int lane = threadIdx.x;
@@ -1411,90 +1435,101 @@ __global__ void __launch_bounds__(64) dx_dense_kernel(DxK p, const float* __rest
     hi = a;
   }
   const int tok0 = tc * 64 * T + T * lane;
-  __shared__ uint2 st[64];  // (record, weight bits) of the chunk's edges
-  // per feature of the range, every lane's T sums: lane-major rows of T floats (no bank conflicts)
-  __shared__ float sums[FW][64 * T];
+  float acc[FW][T];
 #pragma unroll
   for (int x = 0; x < FW; ++x)
 #pragma unroll
-    for (int j = 0; j < T; ++j) sums[x][T * lane + j] = 0.f;
+    for (int j = 0; j < T; ++j) acc[x][j] = 0.f;
   float r[T];  // the open run: its feature fc (wave-uniform; -1 before the first edge)
 #pragma unroll
   for (int j = 0; j < T; ++j) r[j] = 0.f;
   int fc = -1;
-  const unsigned lo8 = (unsigned)tok0 * 4u;  // the lane's byte offset in a dz row
-  for (int si = lo; si < hi; ++si) {
-    const int u = p.seg_unit[si];
-    const long long nb = pool_base(u / p.P, p.S, p.sps, p.gs) + (long long)(u % p.P) * US;  // first neuron of the unit
-    const unsigned e_end = p.seg_begin[si + 1];
-    for (unsigned e0 = p.seg_begin[si]; e0 < e_end; e0 += 64) {
-      const int n = (int)min(e_end - e0, 64u);
-      if (lane < n) {
-        const unsigned rec = p.rec[e0 + lane];
-        const float wv = ld_param(p.W, p.wbf, nb * K + (long long)((rec & REC_OFF_MASK) >> 2));
-        st[lane] = make_uint2(rec, __float_as_uint(wv));
+  const unsigned vo = tok0 < p.Bc ? (unsigned)tok0 * 4u : 0x80000000u;  // the lane's byte offset in a dz row
+  const unsigned rb = (unsigned)p.cap * 4u;                              // bytes of a dz row
+  // edges whose rows are in flight together, in two alternating batches (T = 4: 12.6M neurons, 256
+  // tokens, 4096 inputs 10.6 ms with 2, 11.4 with 4, 11.4 held to 96 VGPRs for a fifth wave)
+  constexpr int DB = T == 4 ? 2 : (T == 2 ? 4 : 8);
+  if (lo < hi) {
+    DxChunk cc{lo, p.seg_begin[lo], p.seg_begin[lo + 1], p.seg_unit[lo]};
+    unsigned pe = 0u, pu = 0u;
+    dx_seg_ahead(p, lo, hi, pe, pu);
+    unsigned rec = dx_load_rec(p, cc, lane);
+    for (;;) {
+      const int n = (int)min(cc.end - cc.e, 64u);
+      const long long nb = pool_base(cc.u / p.P, p.S, p.sps, p.gs) + (long long)(cc.u % p.P) * US;  // first neuron of the unit
+      const unsigned woff = rec & REC_OFF_MASK;
+      float wv;
+      if (p.wbf) {
+        const unsigned boff = woff >> 1;
+        wv = bf16_half(ld_uniform_u32(reinterpret_cast<const unsigned short*>(p.W) + nb * K, boff & ~3u), boff);
+      } else {
+        wv = __uint_as_float(ld_uniform_u32(p.W + nb * K, woff));
       }
-      __syncthreads();
-      // DB edges at a time: their dz rows are loaded together (DB loads in flight per wave, where
-      // one dependent load per edge exposed each load's latency), then added in edge order.  With
-      // the unit-range passes most rows come from the caches, and fewer rows in flight (fewer
-      // VGPRs, more waves) pay: at 2 tokens per lane (C2, 128-token chunks) 3.63 / 3.37 / 3.24 /
-      // 3.40 ms per pass for DB = 8 / 4 / 3 / 2; at 4 tokens per lane (C5 shape) DB = 4 3.58 ms, 2 3.99
-      constexpr int DB = T == 4 ? 4 : (T == 2 ? 3 : 8);
-      for (int i0 = 0; i0 < n; i0 += DB) {
-        float v[DB][T], wv[DB];
-        int f[DB];
+      const __amdgpu_buffer_rsrc_t rows = uniform_rsrc(dz + nb * p.cap);
+      const int off = (int)((woff >> (K == 8 ? 5 : 6)) * rb);
+      const int f = (int)((rec >> REC_F_SHIFT) & REC_F_MASK);
+      const int fp = __builtin_amdgcn_update_dpp(fc, f, 0x138, 0xf, 0xf, false);  // wave_shr:1, lane 0 takes fc
+      const unsigned long long starts = __builtin_amdgcn_ballot_w64(lane < n && f != fp);
+      auto load = [&](int i0, float(&v)[DB][T]) {
+        if (i0 >= n) return;
 #pragma unroll
-        for (int u = 0; u < DB; ++u) {
-          const int i = i0 + u < n ? i0 + u : n - 1;  // past the chunk: the last edge again, not added
-          uint2 e = st[i];
-          e.x = __builtin_amdgcn_readfirstlane(e.x);  // the same edge in every lane
-          e.y = __builtin_amdgcn_readfirstlane(e.y);
-          f[u] = i0 + u < n ? (int)((e.x >> REC_F_SHIFT) & REC_F_MASK) : FW;
-          const long long nn = nb + ((e.x & REC_OFF_MASK) >> (K == 8 ? 5 : 6));
-          wv[u] = __uint_as_float(e.y);
-          const float* row = dz + nn * p.cap;  // scalar row base (buffer resource), the lane's 32-bit offset
+        for (int u = 0; u < DB; ++u) {  // (past the chunk: rows of its first edge, not added)
+          const int so = __builtin_amdgcn_readlane(off, (i0 + u) & 63);
           if constexpr (T == 4) {
-            const uint4 x = ld_uniform_u128(row, lo8);
-            v[u][0] = __uint_as_float(x.x), v[u][1] = __uint_as_float(x.y);
-            v[u][2] = __uint_as_float(x.z), v[u][3] = __uint_as_float(x.w);
+            const auto x = __builtin_amdgcn_raw_buffer_load_b128(rows, (int)vo, so, 0);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[u][j] = __uint_as_float(x[j]);
           } else if constexpr (T == 2) {
-            const uint2 x = ld_uniform_u64(row, lo8);
-            v[u][0] = __uint_as_float(x.x), v[u][1] = __uint_as_float(x.y);
+            const auto x = __builtin_amdgcn_raw_buffer_load_b64(rows, (int)vo, so, 0);
+            v[u][0] = __uint_as_float(x[0]), v[u][1] = __uint_as_float(x[1]);
           } else {
-            v[u][0] = __uint_as_float(ld_uniform_u32(row, lo8));
+            v[u][0] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rows, (int)vo, so, 0));
           }
         }
+      };
+      auto add = [&](int i0, const float(&v)[DB][T]) {
 #pragma unroll
         for (int u = 0; u < DB; ++u) {
-          if (f[u] >= FW) break;  // past the chunk (uniform)
-          if (f[u] != fc) {       // the run ends: add it to its feature's sums
-            if (fc >= 0) {
-#pragma unroll
-              for (int j = 0; j < T; ++j) sums[fc][T * lane + j] += r[j];
-            }
-            fc = f[u];
+          const int i = i0 + u;
+          if (i >= n) return;
+          if ((starts >> i) & 1) {  // a run ends: add it to its feature's sums
+            dx_add_run<0, T>(fc, r, acc);
+            fc = __builtin_amdgcn_readlane(f, i);
 #pragma unroll
             for (int j = 0; j < T; ++j) r[j] = 0.f;
           }
+          const float w = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(wv), i));
 #pragma unroll
-          for (int j = 0; j < T; ++j) r[j] = __builtin_fmaf(wv[u], v[u][j], r[j]);
+          for (int j = 0; j < T; ++j) r[j] = __builtin_fmaf(w, v[u][j], r[j]);
         }
+      };
+      float va[DB][T], vb[DB][T];
+      load(0, va);
+      // the next chunk's records land while this chunk is added; the segment table is read a chunk
+      // ahead, so nothing here waits behind the rows just requested
+      DxChunk cn = cc;
+      dx_next_ahead(p, cn, hi, pe, pu);
+      const bool more = cn.si < hi;
+      const unsigned rn = more ? dx_load_rec(p, cn, lane) : 0u;
+      for (int i0 = 0; i0 < n; i0 += 2 * DB) {
+        load(i0 + DB, vb);
+        add(i0, va);
+        load(i0 + 2 * DB, va);
+        add(i0 + DB, vb);
       }
-      __syncthreads();
+      if (!more) break;
+      cc = cn;
+      rec = rn;
     }
   }
-  if (fc >= 0) {
-#pragma unroll
-    for (int j = 0; j < T; ++j) sums[fc][T * lane + j] += r[j];
-  }
+  dx_add_run<0, T>(fc, r, acc);
   float* out = p.part + (long long)q * p.D * p.cap;
 #pragma unroll
   for (int x = 0; x < FW; ++x) {
     const int d = F * FW + x;
     if (d < p.D) {
 #pragma unroll
-      for (int j = 0; j < T; ++j) out[(long long)d * p.cap + tok0 + j] = sums[x][T * lane + j];
+      for (int j = 0; j < T; ++j) out[(long long)d * p.cap + tok0 + j] = acc[x][j];
     }
   }
 }
@@ -1924,6 +1959,7 @@ extern "C" int gl_bwd(const GlBwdArgs* a, void* stream) {
              (const int32_t*)(eb + h.off_seg_unit), (const uint32_t*)(eb + h.off_seg_begin), c1t, nullptr, W, part,
              NS, a->D, a->S, q.P, q.U, q.QL, q.UQs, q.FR, cap, cap / (64 * Td), sps, gs};
       dk.wbf = wbf;
+      dk.Bc = Bc;
       for (int ql0 = 0; ql0 < q.QLs; ql0 += q.QL) {  // passes of QL unit ranges per XCD
         dk.ql0 = ql0;
         GL_TRY(launch_dx_dense(a->K, Td, dk, dz, s));

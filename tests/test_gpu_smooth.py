@@ -216,3 +216,33 @@ def test_power_mean_integer_p(case, p):
     assert_parity(dx, wdX, mX, what=f"p {p} dX")
     assert_parity(dw.cpu().numpy().reshape(-1, L.fan_in), wdW, mW, what=f"p {p} dW")
     assert_parity(db.cpu().numpy().reshape(-1), wdb, mb, what=f"p {p} db")
+
+
+# the dense dX at its edges: one feature range (D = 16, 24), segments of one edge to several 64-edge
+# chunks (pools of 9 to 1100 slots), tokens around the 64 / 128 / 256-token slices, bf16 weights
+DENSE_DX_EDGES = [
+    # D, H, G, K, B, w dtype
+    (16, 9, 1, 8, 1, torch.float32),
+    (24, 330, 30, 16, 63, torch.float32),
+    (17, 2200, 2, 8, 64, torch.bfloat16),
+    (700, 900, 60, 8, 65, torch.float32),
+    (40, 1100, 1, 16, 127, torch.bfloat16),
+    (333, 3001, 3, 8, 129, torch.float32),
+    (64, 500, 5, 8, 257, torch.float32),
+]
+
+
+@pytest.mark.parametrize("case", DENSE_DX_EDGES, ids=lambda c: f"D{c[0]}H{c[1]}K{c[3]}B{c[4]}{str(c[5])[6:]}")
+def test_dense_dx_at_segment_and_token_edges(case):
+    D, H, G, K, B, wdt = case
+    L, idx, w, b, x, dy = _case((D, H, G, K, B, torch.float32), seed=D)
+    w = w.to(wdt)
+    rt = Level1Runtime(L, idx.to(DEV), _spec("softmax_weighted", 1.0, "identity"), PhysicalPlan())
+    xd, wd, bd = x.to(DEV), w.to(DEV), b.to(wdt).to(DEV)
+    out = rt.forward(xd, wd, bd)
+    dw, db = torch.zeros(L.weight_shape, device=DEV), torch.zeros(L.bias_shape, device=DEV)
+    dx = rt.backward(xd, wd, bd, dy.to(DEV), out, "minimal_stats", dw, db).cpu().numpy()
+    fi, fw, fb = _flat(L, idx, w.float(), b.to(wdt).float())
+    _, _, wdX, (_, _, mX) = O.backward_smooth(x.numpy(), fi, fw, fb, L.counts_tensor("cpu").numpy(), L.slots_per_group,
+                                              dy.numpy(), "softmax_weighted", 1.0, "identity")
+    assert_parity(dx, wdX, mX, what="dX")
