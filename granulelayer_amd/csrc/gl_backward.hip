@@ -556,6 +556,20 @@ struct DxGather {
   unsigned m[2 * T];
 };
 
+// Pool and first neuron of unit u.  FLAT: one unit per pool and pools back to back (P = 1, and shards
+// that fill their groups): pool u starts at neuron u S, where the general form takes two scalar
+// divisions (~16 instructions each, per chunk of a few edges).
+template <bool FLAT>
+__device__ __forceinline__ int unit_pool(const DxK& p, int u) {
+  if constexpr (FLAT) return u;
+  else return u / p.P;
+}
+template <bool FLAT>
+__device__ __forceinline__ long long unit_base(const DxK& p, int u) {
+  if constexpr (FLAT) return (long long)u * p.S;
+  else return pool_base(u / p.P, p.S, p.sps, p.gs) + (long long)(u % p.P) * US;
+}
+
 struct DxChunk {
   int si;           // segment index
   unsigned e, end;  // chunk begin, segment end (edge positions)
@@ -582,10 +596,10 @@ __device__ __forceinline__ unsigned dx_load_rec(const DxK& p, const DxChunk& c, 
   return ld_uniform_u32(p.rec + c.e, (unsigned)lane < n ? (unsigned)lane * 4u : 0u);
 }
 
-template <int K, int T>
+template <int K, int T, bool FLAT>
 __device__ __forceinline__ void dx_gather(const DxK& p, const uint32_t* mask_tc, const DxChunk& c, unsigned rec,
                                           DxGather<T>& g) {
-  const long long nb = pool_base(c.u / p.P, p.S, p.sps, p.gs) + (long long)(c.u % p.P) * US;  // first neuron of the unit
+  const long long nb = unit_base<FLAT>(p, c.u);  // first neuron of the unit
   const unsigned woff = rec & REC_OFF_MASK;  // byte offset of W[n, k] in the unit
   const unsigned nl = woff >> (K == 8 ? 5 : 6);
   g.rec = rec;
@@ -612,9 +626,9 @@ __device__ __forceinline__ void dx_gather(const DxK& p, const uint32_t* mask_tc,
 }
 
 // c1 of the lane's T tokens (tok0 = the first of them) for the pool of unit u
-template <int T>
+template <int T, bool FLAT>
 __device__ __forceinline__ void dx_load_c1(const DxK& p, int u, int tok0, float (&c1)[T]) {
-  const float* c = p.c1t + (long long)(u / p.P) * p.cap + tok0;
+  const float* c = p.c1t + (long long)unit_pool<FLAT>(p, u) * p.cap + tok0;
   if constexpr (T == 4) {
     const float4 v = *reinterpret_cast<const float4*>(c);
     c1[0] = v.x, c1[1] = v.y, c1[2] = v.z, c1[3] = v.w;
@@ -703,7 +717,31 @@ __device__ __forceinline__ void dx_compute(const DxGather<T>& g, DxStage<T>& st,
   __syncthreads();  // the next chunk's staging overwrites st
 }
 
-template <int K, int T>
+// dx_next with the segment table read one step ahead: (pe, pu) hold the end and the unit of
+// segment c.si + 1, loaded by the step that entered segment c.si; their loads land by the next
+// loop-top wait, so no wait for them sits behind a chunk copy
+__device__ __forceinline__ void dx_seg_ahead(const DxK& p, int si, int hi, unsigned& pe, unsigned& pu) {
+  if (si + 1 < hi) {  // 32-bit vector offsets from the tables' bases: no 64-bit scalar address arithmetic
+    const unsigned o = (unsigned)opaque(si * 4);
+    pe = *reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(p.seg_begin) + (o + 8u));
+    pu = *reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(p.seg_unit) + (o + 4u));
+  }
+}
+__device__ __forceinline__ void dx_next_ahead(const DxK& p, DxChunk& c, int hi, unsigned& pe, unsigned& pu) {
+  if (c.e + 64 < c.end) {
+    c.e += 64;
+  } else {
+    c.si += 1;
+    if (c.si < hi) {
+      c.e = c.end;
+      c.end = __builtin_amdgcn_readfirstlane(pe);
+      c.u = __builtin_amdgcn_readfirstlane((int)pu);
+      dx_seg_ahead(p, c.si, hi, pe, pu);
+    }
+  }
+}
+
+template <int K, int T, bool FLAT>
 __global__ void __launch_bounds__(64) dx_kernel(DxK p) {
   const int lane = threadIdx.x;
   // Workgroups are dispatched round-robin over the 8 XCDs.  All feature ranges of one unit range
@@ -752,9 +790,9 @@ __global__ void __launch_bounds__(64) dx_kernel(DxK p) {
   if (lo < hi) {
     DxChunk cc{lo, p.seg_begin[lo], p.seg_begin[lo + 1], p.seg_unit[lo]};
     DxGather<T> gc;
-    dx_gather<K, T>(p, mask_tc, cc, dx_load_rec(p, cc, lane), gc);
+    dx_gather<K, T, FLAT>(p, mask_tc, cc, dx_load_rec(p, cc, lane), gc);
     float c1[T];
-    dx_load_c1<T>(p, cc.u, tok0, c1);
+    dx_load_c1<T, FLAT>(p, cc.u, tok0, c1);
     DxChunk cn = cc;
     dx_next(p, cn, hi);
     unsigned rn = cn.si < hi ? dx_load_rec(p, cn, lane) : 0u;
@@ -769,8 +807,8 @@ __global__ void __launch_bounds__(64) dx_kernel(DxK p) {
       DxChunk cnn = cn;
       unsigned rnn = 0u;
       if (more) {
-        dx_gather<K, T>(p, mask_tc, cn, rn, gn);
-        if (cn.si != cc.si) dx_load_c1<T>(p, cn.u, tok0, c1n);
+        dx_gather<K, T, FLAT>(p, mask_tc, cn, rn, gn);
+        if (cn.si != cc.si) dx_load_c1<T, FLAT>(p, cn.u, tok0, c1n);
         dx_next(p, cnn, hi);
         if (cnn.si < hi) rnn = dx_load_rec(p, cnn, lane);
       }
@@ -816,9 +854,9 @@ constexpr int DX_SLICE_WORDS = 2 * 65 * 4;
 
 // the chunk's weights and the NS slices' mask rows -> buffer buf (lanes past the chunk copy the
 // first edge's); slice s reads slab tc0 + s of the mask
-template <int K, int NS>
+template <int K, int NS, bool FLAT>
 __device__ __forceinline__ void dx_dma(const DxK& p, int tc0, const DxChunk& c, unsigned rec, DxDma<NS>& st, int buf) {
-  const long long nb = pool_base(c.u / p.P, p.S, p.sps, p.gs) + (long long)(c.u % p.P) * US;  // first neuron of the unit
+  const long long nb = unit_base<FLAT>(p, c.u);  // first neuron of the unit
   const unsigned woff = rec & REC_OFF_MASK;  // byte offset of W[n, k] in the unit
   const unsigned mo = (woff >> (K == 8 ? 5 : 6)) * 32u;  // byte offset of the neuron's mask row
   // bf16 W: the 32-bit word holding the weight (its half is taken when the chunk is read)
@@ -839,8 +877,8 @@ __device__ __forceinline__ void dx_dma(const DxK& p, int tc0, const DxChunk& c, 
   }
 }
 
-// dx_run over the DMA layout: mrow = the lane's mask word of edge 0 in slice 0 (rows 16 bytes
-// apart, slice s DX_SLICE_WORDS further); wl = the weight of the lane's own edge, edge i's weight
+// dx_run over the DMA layout, edges i .. i1 - 1: mrow = LDS address of the lane's mask word of edge 0 in
+// slice 0 (rows 16 bytes apart, slice s DX_SLICE_WORDS further); wl = the weight of the lane's own edge, edge i's weight
 // taken from lane i (v_readlane, one VALU instead of one more LDS read per edge)
 template <int X, int NS>
 __device__ __forceinline__ void dx_run_dma(const unsigned* mrow, float wl, const float (*lut)[4], int i0, int i1,
@@ -886,42 +924,19 @@ __device__ __forceinline__ void dx_runs_dma(const unsigned* mrow, float wl, cons
   if constexpr (X + 1 < FW) dx_runs_dma<X + 1, NS>(mrow, wl, lut, b, bit, c1, acc);
 }
 
-// dx_next with the segment table read one step ahead: (pe, pu) hold the end and the unit of
-// segment c.si + 1, loaded by the step that entered segment c.si; their loads land by the next
-// loop-top wait, so no wait for them sits behind a chunk copy
-__device__ __forceinline__ void dx_seg_ahead(const DxK& p, int si, int hi, unsigned& pe, unsigned& pu) {
-  if (si + 1 < hi) {
-    pe = p.seg_begin[si + 2];
-    pu = (unsigned)p.seg_unit[si + 1];
-  }
-}
-__device__ __forceinline__ void dx_next_ahead(const DxK& p, DxChunk& c, int hi, unsigned& pe, unsigned& pu) {
-  if (c.e + 64 < c.end) {
-    c.e += 64;
-  } else {
-    c.si += 1;
-    if (c.si < hi) {
-      c.e = c.end;
-      c.end = __builtin_amdgcn_readfirstlane(pe);
-      c.u = __builtin_amdgcn_readfirstlane((int)pu);
-      dx_seg_ahead(p, c.si, hi, pe, pu);
-    }
-  }
-}
-
 // c1 of the lane's 4 tokens of each of the NS slices for the pool of unit u: a uniform row base
 // (scalar registers) plus the lane's 32-bit offset (no 64-bit vector address to keep live)
-template <int NS>
+template <int NS, bool FLAT>
 __device__ __forceinline__ void dx_load_c1_u(const DxK& p, int u, int slice0, int lane, float (&c1)[NS][4]) {
 #pragma unroll
   for (int sl = 0; sl < NS; ++sl) {
-    const uint4 v = ld_uniform_u128(p.c1t + (long long)(u / p.P) * p.cap + slice0 + sl * 256, (unsigned)lane * 16u);
+    const uint4 v = ld_uniform_u128(p.c1t + (long long)unit_pool<FLAT>(p, u) * p.cap + slice0 + sl * 256, (unsigned)lane * 16u);
     c1[sl][0] = __uint_as_float(v.x), c1[sl][1] = __uint_as_float(v.y), c1[sl][2] = __uint_as_float(v.z),
     c1[sl][3] = __uint_as_float(v.w);
   }
 }
 
-template <int K, int NS>
+template <int K, int NS, bool FLAT>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(NS == 1 ? 8 : 4, NS == 1 ? 8 : 4)))
 dx_dma_kernel(DxK p) {
   constexpr int T = 4;
@@ -975,10 +990,10 @@ dx_dma_kernel(DxK p) {
     dx_next_ahead(p, cn, hi, pe, pu);
     const unsigned rc0 = dx_load_rec(p, cc, lane);
     unsigned rn = cn.si < hi ? dx_load_rec(p, cn, lane) : 0u;
-    dx_dma<K, NS>(p, tc0, cc, rc0, st, 0);
+    dx_dma<K, NS, FLAT>(p, tc0, cc, rc0, st, 0);
     unsigned rc = rc0;
     float c1[NS][T];
-    dx_load_c1_u<NS>(p, cc.u, tc0 * 64 * T, lane, c1);
+    dx_load_c1_u<NS, FLAT>(p, cc.u, tc0 * 64 * T, lane, c1);
     int cur = 0;
     for (;;) {
       // every copy, load and LDS read so far is done: buffer cur holds chunk cc, and buffer
@@ -997,8 +1012,8 @@ dx_dma_kernel(DxK p) {
         // the copy (the counter is in order); their values were loaded one step ago
         dx_next_ahead(p, cnn, hi, pe, pu);
         if (cnn.si < hi) rnn = dx_load_rec(p, cnn, lane);
-        dx_dma<K, NS>(p, tc0, cn, rn, st, cur ^ 1);
-        if (cn.si != cc.si) dx_load_c1_u<NS>(p, cn.u, tc0 * 64 * T, lane, c1n);
+        dx_dma<K, NS, FLAT>(p, tc0, cn, rn, st, cur ^ 1);
+        if (cn.si != cc.si) dx_load_c1_u<NS, FLAT>(p, cn.u, tc0 * 64 * T, lane, c1n);
       }
       {
         const int n = (int)min(cc.end - cc.e, 64u);
@@ -1406,7 +1421,7 @@ __device__ __forceinline__ void dx_add_run(int f, const float (&r)[T], float (&a
 // LogMeanExp dX before -> now: 4M neurons, 64 tokens, 1024 inputs 1.82 -> 0.88 ms; 0.78M at fan-in 16,
 // 77 tokens, 1000 inputs 731 -> 535 us; 2M, 200 tokens, 8000 inputs 3.00 -> 1.96 ms; 12.6M, 256
 // tokens, 4096 inputs 11.3 -> 10.6 ms (there the 103 GB of row reads bound it: 9.8 TB/s).
-template <int K, int T>
+template <int K, int T, bool FLAT>
 __global__ void __launch_bounds__(64) dx_dense_kernel(DxK p, const float* __restrict__ dz) {
   const int lane = threadIdx.x;
   const int bid = blockIdx.x;
@@ -1456,7 +1471,7 @@ __global__ void __launch_bounds__(64) dx_dense_kernel(DxK p, const float* __rest
     unsigned rec = dx_load_rec(p, cc, lane);
     for (;;) {
       const int n = (int)min(cc.end - cc.e, 64u);
-      const long long nb = pool_base(cc.u / p.P, p.S, p.sps, p.gs) + (long long)(cc.u % p.P) * US;  // first neuron of the unit
+      const long long nb = unit_base<FLAT>(p, cc.u);  // first neuron of the unit
       const unsigned woff = rec & REC_OFF_MASK;
       float wv;
       if (p.wbf) {
@@ -1751,19 +1766,28 @@ static int launch_bwd_w_any(int K, int act, const BwK& k, hipStream_t s) {
   return act == GL_ACT_RELU ? launch_bwd_w_act<GL_ACT_RELU>(K, k, s) : launch_bwd_w_act<GL_ACT_IDENTITY>(K, k, s);
 }
 
+// Flat units (unit_pool): a chunk of a dX wave is one pool's few edges into 8 inputs, and its scalar
+// control, with two divisions among ~200 scalar instructions, bounds the kernels where segments are
+// short (a scalar instruction issues every 4 clocks and SIMD).  Division -> flat, with the segment
+// table read at vector offsets: pools of 256 as shards, 12.6M neurons, 256 tokens, 4096 inputs (4 edges
+// a segment) 6.44 -> 4.19 ms; 1M, 64 tokens, 1024 inputs 197 -> 173 us; 25M, 256 tokens, 4096 inputs
+// 4.60 -> 4.30 ms; 100M, 1024 tokens, 8192 inputs 92.1 -> 88.7 ms; 256-wide windows 3.82 -> 3.67 ms.
+static bool dx_flat(const DxK& k) { return k.P == 1 && (k.sps <= 1 || k.gs == k.sps * k.S); }
+
 template <int K, int T>
 static int launch_dx_kt(const DxK& k, hipStream_t s, bool dma) {
   if constexpr (T == 4) {
     if (dma) {  // two 256-token slices per wave when the chunk has an even number of them
       const bool two = k.n_tc % 2 == 0 && DX_DMA_TWO_SLICES;
-      auto fn = two ? dx_dma_kernel<K, 2> : dx_dma_kernel<K, 1>;
+      auto fn = dx_flat(k) ? (two ? dx_dma_kernel<K, 2, true> : dx_dma_kernel<K, 1, true>)
+                           : (two ? dx_dma_kernel<K, 2, false> : dx_dma_kernel<K, 1, false>);
       GL_LAUNCH(GL_KERNEL_DX_DMA, fn, dim3((unsigned)(8LL * k.FR * k.QL * (two ? k.n_tc / 2 : k.n_tc))), dim3(64), 0,
                 s, k);
       GL_CHECK_LAUNCH();
       return 0;
     }
   }
-  auto fn = dx_kernel<K, T>;
+  auto fn = dx_flat(k) ? dx_kernel<K, T, true> : dx_kernel<K, T, false>;
   GL_LAUNCH(GL_KERNEL_DX, fn, dim3((unsigned)(8LL * k.FR * k.QL * k.n_tc)), dim3(64), 0, s, k);
   GL_CHECK_LAUNCH();
   return 0;
@@ -1821,7 +1845,8 @@ static int launch_bwd_smooth_kk(int pool, int act, const BsK& k, hipStream_t s) 
 
 template <int K, int T>
 static int launch_dx_dense_kt(const DxK& k, const float* dz, hipStream_t s) {
-  GL_LAUNCH(GL_KERNEL_DX_DENSE, (dx_dense_kernel<K, T>), dim3((unsigned)(8LL * k.FR * k.QL * k.n_tc)), dim3(64), 0, s, k,
+  auto fn = dx_flat(k) ? dx_dense_kernel<K, T, true> : dx_dense_kernel<K, T, false>;
+  GL_LAUNCH(GL_KERNEL_DX_DENSE, fn, dim3((unsigned)(8LL * k.FR * k.QL * k.n_tc)), dim3(64), 0, s, k,
             dz);
   GL_CHECK_LAUNCH();
   return 0;

@@ -180,3 +180,38 @@ def test_max_of_shard_maxima_is_the_flat_maximum_on_the_gpu():
                                   device=DEV, seed=1, bias_std=0.2)
     x = torch.randn(16, 64, generator=torch.Generator().manual_seed(2)).to(DEV)
     assert torch.equal(lay(x).detach(), flat(x).detach())
+
+
+@pytest.mark.parametrize("K,B", [(8, 3), (8, 130), (8, 520), (16, 70)])
+@pytest.mark.parametrize("full", [True, False], ids=["full_shards", "ragged_shards"])
+def test_shard_dx_equals_the_plain_pools(full, K, B):
+    """Shards that fill their groups lie back to back like plain pools of their size (the dX kernels'
+    flat units): dX, dW and db of the same neurons as 4 shards per group and as 4 G pools agree bit for
+    bit.  With a last shard that ends inside the group the units take the general form; the same pools
+    exist as plain layout pools of unequal size only, so there the oracle's bar on dX applies."""
+    G, nps, D = 6, 64, 200
+    per = 4 * nps if full else 4 * nps - 32
+    L = SparseLayout(D, G * per, G, K, 8, False)
+    idx, w, b = init_parameters(L, "cpu", torch.float32, seed=K + B, bias_std=0.3)
+    gen = torch.Generator().manual_seed(B)
+    x, dy = torch.randn(B, D, generator=gen).to(DEV), torch.randn(B, 4 * G, generator=gen)
+
+    def backward(layout, i, wt, bt, nps_):
+        rt = Level1Runtime(layout, i.to(DEV), LevelSpec("sum", activation="relu"), PhysicalPlan(), nps_)
+        dw, db = torch.zeros(layout.weight_shape, device=DEV), torch.zeros(layout.bias_shape, device=DEV)
+        dx = rt.backward(x, wt.to(DEV), bt.to(DEV), dy.to(DEV), {}, "minimal_stats", dw, db)
+        return dx, dw.reshape(-1), db.reshape(-1)
+
+    got = backward(L, idx, w, b, nps)
+    if full:
+        P = SparseLayout(D, G * per, 4 * G, K, 8, False)
+        want = backward(P, idx.view(P.index_shape), w.view(P.weight_shape), b.view(P.bias_shape), None)
+        for name, a, c in zip(("dX", "dW", "db"), got, want):
+            assert torch.equal(a, c), name
+        return
+    counts = np.array([nps, nps, nps, nps - 32] * G, np.int32)  # oracle pools of nps slots, the last ones padded
+    fi, fw, fb = (t.reshape(G, per, -1).numpy() for t in (idx, w, b))
+    pad = ((0, 0), (0, 32), (0, 0))
+    fi, fw, fb = (np.pad(t, pad).reshape(G * 4 * nps, -1) for t in (fi, fw, fb))
+    _, _, dX, bnd = O.backward(x.cpu().numpy(), fi, fw, fb[:, 0], counts, nps, dy.numpy(), "relu", "sum", with_bounds=True)
+    assert_parity(got[0].cpu().numpy(), dX, bnd["mag"][2], bnd["unc"][2], what="dX")
