@@ -791,9 +791,11 @@ __device__ __forceinline__ void fwd_tile_dispatch(SRC xsb, const unsigned (&addr
 template <int K, int NPL, int WAVES, int ACT, bool DBUF, bool WS = false, int PK = PK_SUM, bool XG = false,
           bool SMALL = false, int TB = BT, bool XB = false, bool FM = false>
 // SMALL: two workgroups share a CU, so a wave must fit 128 VGPRs (4 waves per SIMD)
-__global__ void __launch_bounds__(WAVES * 64, SMALL ? 16 / WAVES * WAVES / 4 : 1) fwd_kernel(FwdK p) {
+__global__ void __launch_bounds__(WAVES * 64, SMALL ? (K == 16 && PK != PK_SUM ? 2 : (WAVES == 12 ? 3 : 16 / WAVES * WAVES / 4)) : 1)
+    fwd_kernel(FwdK p) {
   // WS: xa holds both stage regions (2 * WS_TILES * nsl <= 2 * XTILE_DB slots, XTILE_DB with
-  // SMALL); XG: no LDS tile; SMALL: one single-buffered tile of at most XTILE_DB 16-byte slots, so
+  // SMALL); WS with SMALL for the other pools than sum / mean: stages of whole narrow tiles (12 waves:
+  // in 2 * XTILE_DB slots); XG: no LDS tile; SMALL: one single-buffered tile of at most XTILE_DB 16-byte slots, so
   // two workgroups share a CU.  TB: tokens per tile (4, or 2 for the two-token tiles of DBUF sum /
   // mean: D x 8 bytes per buffer)
   // XB: 4-token tiles of raw bf16 (8-byte slots, bf16 X), one buffer (SMALL) or two
@@ -801,7 +803,7 @@ __global__ void __launch_bounds__(WAVES * 64, SMALL ? 16 / WAVES * WAVES / 4 : 1
   static_assert(!XB || (TB == BT && (DBUF || SMALL || WS) && !XG && PK == PK_SUM), "bf16 tiles: sum / mean");
   static_assert(!FM || (TB == BT && PK == PK_SUM && ACT == GL_ACT_RELU), "ReLU bits: 4-token tiles, sum / mean");
   constexpr int SLOT = XB ? 8 : 4 * TB;  // bytes per input of a tile or stage
-  __shared__ float4 xa[WS ? (SMALL ? XTILE_DB : 2 * XTILE_DB) : (XG ? 1 : (DBUF || SMALL ? XTILE_DB : XTILE_SB))];
+  __shared__ float4 xa[WS ? (SMALL && WAVES != 12 ? XTILE_DB : 2 * XTILE_DB) : (XG ? 1 : (DBUF || SMALL ? XTILE_DB : XTILE_SB))];
   __shared__ float4 xb[DBUF ? XTILE_DB : 1];
   // top-k: the ranked tile's per-wave candidate lists, where the CU's LDS has room for them
   constexpr int TKW = PK == PK_TOPK && (SMALL ? 2 : 1) * (sizeof(xa) + sizeof(xb) + WAVES * 4 * TK_CAP * 8) <= 160 * 1024
@@ -829,7 +831,8 @@ __global__ void __launch_bounds__(WAVES * 64, SMALL ? 16 / WAVES * WAVES / 4 : 1
   const int pk = WS && p.win ? (int)(g - g_first) : 0;
   const int lo = WS && p.win ? (int)__builtin_amdgcn_readfirstlane(p.win[g]) : 0;
   // the lane's neurons: input addresses, weights, bias, slots
-  if constexpr (WS) {
+  constexpr bool NARROW = WS && SMALL && PK != PK_SUM;  // whole tiles only (p.win null)
+  if constexpr (WS && !NARROW) {
     // pool windows: the parameter dtype tested per load (the set-up below, written as a generic
     // lambda, added spills to these kernels)
 #pragma unroll
@@ -1229,6 +1232,16 @@ constexpr int fwd_waves(int K, int pk = PK_SUM, int act = GL_ACT_RELU) {
                     act != GL_ACT_GELU;
   return K == 8 ? (pk == PK_SUM ? 16 : (pk == PK_MAX || pk == PK_TOPK || sm12 ? 12 : 8)) : (pk == PK_SUM ? 8 : 4);
 }
+// fan-in 16, LogMeanExp, softmax-weighted, power mean (p = 1, 2, 4) and top-k over at most 2048
+// inputs: whole tiles staged in 64 KiB, so two 4-wave workgroups share a CU (2 waves per SIMD at
+// 244-256 VGPRs) where 128 KiB of buffers leave one wave per SIMD and nothing to hide its latency.
+// 1M neurons: LogMeanExp, 200 tokens, D = 1500 549 -> 418 us; top-8, 64 tokens, D = 500 264 -> 186;
+// power mean, p = 2, 64 tokens, D = 700 193 -> 145; 0.78M softmax-weighted, 77 tokens, D = 1000 216 -> 150.
+// GELU neurons, max, p = 8 and a p read at run time spill 2-200 VGPRs at 256 and keep the two buffers
+// (max 778 -> 975 us).
+constexpr bool fwd_narrow16(int K, int pk, int act) {
+  return K == 16 && act != GL_ACT_GELU && (pk == PK_LME || pk == PK_SW || pk == PK_TOPK || (pk_pint(pk) > 0 && pk_pint(pk) < 8));
+}
 static int pool_kind(int pool) {
   switch (pool) {
     case GL_POOL_MAX: return PK_MAX;
@@ -1338,6 +1351,8 @@ static int launch_fwd_buf(int D, const FwdK& k, hipStream_t s) {
     }
     if constexpr (W % 8 == 0 && !pk_smooth(PK))
       if (k.ws_small) return launch_fwd<K, FWD_NPL, W / 2, ACT, false, true, PK, false, true>(k, s);
+    if constexpr (fwd_narrow16(K, PK, ACT) || (K == 8 && PK == PK_MAX))
+      if (k.ws_small) return launch_fwd<K, FWD_NPL, W, ACT, false, true, PK, false, true>(k, s);
     return launch_fwd<K, FWD_NPL, W, ACT, false, true, PK>(k, s);
   }
   // 8-byte-slot tiles (sum / mean, the host chose the format):
@@ -1504,7 +1519,12 @@ static int fwd_run(const GlFwdArgs* a, void* ws, const FwdPlan& q, hipStream_t s
       // (two workgroups per CU hide the barrier: D = 1024 719 -> 776 us), nor at fan-in 16 (max 778
       // -> 840 us), nor with one tile per region (top-8 at D = 4096 4.92 -> 5.23 ms).
       const int tps = stage_tiles(a->D, 16, XTILE_DB, b_pad / BT);
-      if (tps >= 2) k.tps = tps, k.ww = a->D, k.npw = 1;
+      // (max: the set-up without a dtype test per load, 2.22 -> 2.17 ms; top-k would lose its lists' LDS)
+      if (tps >= 2) k.tps = tps, k.ww = a->D, k.npw = 1, k.ws_small = a->pool == GL_POOL_MAX;
+    } else if (fwd_narrow16(a->K, fwd_pool_kind(a), a->act) && b_pad >= 8 * BT) {
+      // (fewer tiles than 8: the two-buffer kernel starts sooner)
+      const int tps = stage_tiles(a->D, 16, XTILE_DB / 2, b_pad / BT);
+      if (tps) k.tps = tps, k.ww = a->D, k.npw = 1, k.ws_small = 1;
     }
     // fp32 X, sum / mean over full tiles of 4097..8192 inputs: two-token tiles (8-byte slots)
     k.tb = !k.xb && pool_kind(a->pool) == PK_SUM && !k.tps && tiles_of_two(a->D) ? 2 : BT;

@@ -82,3 +82,26 @@ def test_narrow_selection_forward_gives_the_bits_of_the_wide_kernel(case, pool, 
         got.append((out["pre"], out["winner" if pool == "max" else "topk_slot"]))
     for name, a, c in zip(("pre", "ids"), *got):
         assert torch.equal(a, c), name
+
+
+# fan-in 16: two workgroups per CU over whole narrow tiles, at least 8 tiles (29 tokens on), D to 2048
+@pytest.mark.parametrize("pool,kw", [("logmeanexp", {"temperature": 0.5}), ("softmax_weighted", {"beta": 1.0}),
+                                     ("power_mean", {"p": 2.0}), ("topk_mean", {"k": 8})])
+@pytest.mark.parametrize("D,B", [(64, 29), (255, 64), (256, 100), (2048, 33)])
+@pytest.mark.parametrize("wdt", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+def test_narrow_fan_in_16_forward_matches_the_wide_kernel(D, B, pool, kw, wdt):
+    """The same layer with 2049 or more inputs runs the two-buffer kernel: the same z (top-k: the same
+    slots and values bit for bit); the smooth states merge in the same order, their exponentials contracted
+    by the compiler as it sees fit, within 8 roundings of fp32 (2^-21 of the value's scale)."""
+    H, G = 3000, 7
+    got = []
+    for wide in (D, 2049 + D % 5):
+        L, idx, x, w, b = _layer(D, H, G, 16, B, torch.float32, wdt, wide)
+        rt = Level1Runtime(L, idx, LevelSpec(pool, activation="relu", **kw), PhysicalPlan())
+        out = rt.forward(x, w, b, track_ids=True)
+        got.append((out["pre"], out.get("topk_slot")))
+    (a, ia), (c, ic) = got
+    if pool == "topk_mean":
+        assert torch.equal(a, c) and torch.equal(ia, ic)
+    else:
+        assert float((a - c).abs().max()) <= 2.0**-21 * float(c.abs().max())
