@@ -299,7 +299,10 @@ __global__ void __launch_bounds__(WAVES * 64, SMALL ? (WS ? 3 : 4) : 1) bwd_w_ke
   unsigned addr[NPL][K];
   float w[NPL][K], dw[NPL][K];
   float bias[NPL], dbv[NPL];
-  unsigned slot2[(NPL + 1) / 2];  // slots of neurons 2i, 2i+1 within the pool (16 bits each; >= n_g: padding)
+  // slots of neurons 2i, 2i+1 counted from the chunk's first schedule window (16 bits each, whatever the
+  // pool's size; >= n_g - s_w: padding)
+  unsigned slot2[(NPL + 1) / 2];
+  const int s_w = s_lo & ~(SCHED_WIN - 1);
   // window staging: this wave's pool is slot pk of the workgroup's staged pools, window start lo
   const int g_first = (int)((long long)blockIdx.x * WAVES / p.cpg);
   // (whole tiles staged, p.win null: one window of all inputs)
@@ -313,7 +316,7 @@ __global__ void __launch_bounds__(WAVES * 64, SMALL ? (WS ? 3 : 4) : 1) bwd_w_ke
     for (int j = 0; j < NPL; ++j) {
       uint32_t order;
       const int s = sched_slot(p.sched, p.nwin, p.S, g, s_lo, j, lane, order);
-      const unsigned s16 = (unsigned)(s < 0xffff ? s : 0xffff);
+      const unsigned s16 = (unsigned)(s - s_w);
       if (j % 2 == 0) slot2[j / 2] = s16; else slot2[j / 2] |= s16 << 16;
       const bool valid = s < n_g;
       const long long n = pool_base((int)g, p.S, p.sps, p.gs) + (s < ext ? s : ext - 1);  // in bounds; invalid slots masked
@@ -348,7 +351,7 @@ __global__ void __launch_bounds__(WAVES * 64, SMALL ? (WS ? 3 : 4) : 1) bwd_w_ke
       for (int j = 0; j < NPL; ++j) {
         uint32_t order;
         const int s = sched_slot(p.sched, p.nwin, p.S, g, s_lo, j, lane, order);
-        const unsigned s16 = (unsigned)(s < 0xffff ? s : 0xffff);
+        const unsigned s16 = (unsigned)(s - s_w);
         if (j % 2 == 0) slot2[j / 2] = s16; else slot2[j / 2] |= s16 << 16;
         const bool valid = s < n_g;
         const long long n = pool_base((int)g, p.S, p.sps, p.gs) + (s < ext ? s : ext - 1);  // in bounds; invalid slots masked
@@ -489,11 +492,11 @@ __global__ void __launch_bounds__(WAVES * 64, SMALL ? (WS ? 3 : 4) : 1) bwd_w_ke
     }
     // odd word: (word - 1, word) in one row of one slab (mw2 is even); a last even word alone
     const int w0 = word & ~1;
-    uint32_t* mslab = p.mask + ((long long)(w0 / p.mw2) * p.NS + pool_base((int)g, p.S, p.sps, p.gs)) * p.mw2 + w0 % p.mw2;
+    uint32_t* mslab = p.mask + ((long long)(w0 / p.mw2) * p.NS + pool_base((int)g, p.S, p.sps, p.gs) + s_w) * p.mw2 + w0 % p.mw2;
 #pragma unroll
     for (int j = 0; j < NPL; ++j) {
       const int s = (int)((opaque((int)slot2[j / 2]) >> (16 * (j % 2))) & 0xffff);  // address math kept local
-      if (!active || s >= n_g) continue;
+      if (!active || s >= n_g - s_w) continue;
       if (word & 1)
         *reinterpret_cast<uint2*>(mslab + (long long)s * p.mw2) = make_uint2(mwe[j], mw[j]);
       else

@@ -99,6 +99,21 @@ def test_backward_matches_oracle(case, pool, act):
     assert not dw.cpu().numpy().reshape(-1, K)[~valid].any()
 
 
+@pytest.mark.parametrize("case", [(512, 8, "relu"), (1700, 8, "relu"), (700, 16, "identity")], ids=str)
+def test_dx_of_pools_of_more_than_65536_slots(case):
+    """A neuron's slot within its pool exceeds 16 bits: the dW pass must still put its mask words into its
+    own row, which dX reads (two pools of 70,001 and 70,000 slots, narrow and wide staging, fan-in 16)."""
+    D, K, act = case
+    L, idx, w, b, x, dy = make_case(D, 140001, 2, K, 70)
+    rt = runtime(L, idx, "mean", act)
+    dw, db = torch.zeros(L.weight_shape, device=DEV), torch.zeros(L.bias_shape, device=DEV)
+    dx = rt.backward(x.to(DEV), w.to(DEV), b.to(DEV), dy.to(DEV), {}, "minimal_stats", dw, db).cpu().numpy()
+    counts = L.counts_tensor("cpu").numpy()
+    _, _, wdX, bnd = O.backward(x.float().numpy(), *flat(L, idx, w, b), counts, L.slots_per_group, dy.numpy(), act,
+                                "mean", with_bounds=True)
+    assert_parity(dx, wdX, bnd["mag"][2], bnd["unc"][2], what="dX")
+
+
 def make_window_case(D, H, G, K, B, width, seed=0, x_dtype=torch.float32):
     """The C3 index structure: every pool draws its inputs from one contiguous window of `width`
     inputs at a seeded offset (padded slots keep index 0)."""
