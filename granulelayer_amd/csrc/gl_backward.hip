@@ -18,8 +18,11 @@
 
 #include "gl_common.h"
 #include "gl_internal.h"
+#include "gl_segments.h"
 
 namespace gl {
+
+static_assert((MAX_SLOTS + 1) * 4 <= 0xffffffffLL, "a dX wave's segment rows lie at 32-bit byte offsets");
 
 // c1t[g, b] = g_pre[b0 + b, g] * scale_g for b < Bc, zero up to cap (tiled transpose); scale_g =
 // 1 / n_g (mean), 1 / min(n_g, k) (top-k mean), else 1.  Max pooling (winner != null) also
@@ -573,25 +576,6 @@ __device__ __forceinline__ long long unit_base(const DxK& p, int u) {
   else return pool_base(u / p.P, p.S, p.sps, p.gs) + (long long)(u % p.P) * US;
 }
 
-struct DxChunk {
-  int si;           // segment index
-  unsigned e, end;  // chunk begin, segment end (edge positions)
-  int u;            // unit of the segment
-};
-
-__device__ __forceinline__ void dx_next(const DxK& p, DxChunk& c, int hi) {
-  if (c.e + 64 < c.end) {
-    c.e += 64;
-  } else {
-    c.si += 1;
-    if (c.si < hi) {
-      c.e = c.end;
-      c.end = p.seg_begin[c.si + 1];
-      c.u = p.seg_unit[c.si];
-    }
-  }
-}
-
 // record of the lane's edge (lanes past the chunk take the chunk's first edge: in bounds, unused);
 // the chunk's base address is wave-uniform (scalar registers), the lane adds a 32-bit offset
 __device__ __forceinline__ unsigned dx_load_rec(const DxK& p, const DxChunk& c, int lane) {
@@ -720,30 +704,6 @@ __device__ __forceinline__ void dx_compute(const DxGather<T>& g, DxStage<T>& st,
   __syncthreads();  // the next chunk's staging overwrites st
 }
 
-// dx_next with the segment table read one step ahead: (pe, pu) hold the end and the unit of
-// segment c.si + 1, loaded by the step that entered segment c.si; their loads land by the next
-// loop-top wait, so no wait for them sits behind a chunk copy
-__device__ __forceinline__ void dx_seg_ahead(const DxK& p, int si, int hi, unsigned& pe, unsigned& pu) {
-  if (si + 1 < hi) {  // 32-bit vector offsets from the tables' bases: no 64-bit scalar address arithmetic
-    const unsigned o = (unsigned)opaque(si * 4);
-    pe = *reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(p.seg_begin) + (o + 8u));
-    pu = *reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(p.seg_unit) + (o + 4u));
-  }
-}
-__device__ __forceinline__ void dx_next_ahead(const DxK& p, DxChunk& c, int hi, unsigned& pe, unsigned& pu) {
-  if (c.e + 64 < c.end) {
-    c.e += 64;
-  } else {
-    c.si += 1;
-    if (c.si < hi) {
-      c.e = c.end;
-      c.end = __builtin_amdgcn_readfirstlane(pe);
-      c.u = __builtin_amdgcn_readfirstlane((int)pu);
-      dx_seg_ahead(p, c.si, hi, pe, pu);
-    }
-  }
-}
-
 template <int K, int T, bool FLAT>
 __global__ void __launch_bounds__(64) dx_kernel(DxK p) {
   const int lane = threadIdx.x;
@@ -760,21 +720,7 @@ __global__ void __launch_bounds__(64) dx_kernel(DxK p) {
   const int q = ql * 8 + xcd;
   const int u_lo = q * p.UQ;
   const int u_hi = min(u_lo + p.UQ, p.U);
-  int lo = (int)p.seg_ptr[F], hi = (int)p.seg_ptr[F + 1];
-  {
-    int a = lo, b = hi;
-    while (a < b) {
-      int mid = (a + b) >> 1;
-      if (p.seg_unit[mid] < u_lo) a = mid + 1; else b = mid;
-    }
-    lo = a;
-    b = hi;
-    while (a < b) {
-      int mid = (a + b) >> 1;
-      if (p.seg_unit[mid] < u_hi) a = mid + 1; else b = mid;
-    }
-    hi = a;
-  }
+  const DxSegs sg = dx_segs(p.seg_ptr, p.seg_unit, p.seg_begin, F, u_lo, u_hi);
   float acc[FW][T];
 #pragma unroll
   for (int f = 0; f < FW; ++f)
@@ -790,19 +736,19 @@ __global__ void __launch_bounds__(64) dx_kernel(DxK p) {
 #pragma unroll
     for (int j = 0; j < T; ++j) st.lut[lane][j] = (lane >> j) & 1 ? 1.0f : 0.0f;
   }
-  if (lo < hi) {
-    DxChunk cc{lo, p.seg_begin[lo], p.seg_begin[lo + 1], p.seg_unit[lo]};
+  if (sg.n > 0) {
+    DxChunk cc = dx_first(sg);
     DxGather<T> gc;
     dx_gather<K, T, FLAT>(p, mask_tc, cc, dx_load_rec(p, cc, lane), gc);
     float c1[T];
     dx_load_c1<T, FLAT>(p, cc.u, tok0, c1);
     DxChunk cn = cc;
-    dx_next(p, cn, hi);
-    unsigned rn = cn.si < hi ? dx_load_rec(p, cn, lane) : 0u;
+    dx_next(sg, cn);
+    unsigned rn = cn.si < sg.n ? dx_load_rec(p, cn, lane) : 0u;
     for (;;) {
       // next chunk: gather (its records were requested one iteration ago), then request the
       // records of the chunk after it; both are in flight while the current chunk is computed
-      const bool more = cn.si < hi;
+      const bool more = cn.si < sg.n;
       DxGather<T> gn = gc;
       float c1n[T];
 #pragma unroll
@@ -812,8 +758,8 @@ __global__ void __launch_bounds__(64) dx_kernel(DxK p) {
       if (more) {
         dx_gather<K, T, FLAT>(p, mask_tc, cn, rn, gn);
         if (cn.si != cc.si) dx_load_c1<T, FLAT>(p, cn.u, tok0, c1n);
-        dx_next(p, cnn, hi);
-        if (cnn.si < hi) rnn = dx_load_rec(p, cnn, lane);
+        dx_next(sg, cnn);
+        if (cnn.si < sg.n) rnn = dx_load_rec(p, cnn, lane);
       }
       dx_compute<T>(gc, st, (int)min(cc.end - cc.e, 64u), lane, word, bit, c1, acc);
       if (!more) break;
@@ -955,21 +901,7 @@ dx_dma_kernel(DxK p) {
   const int q = ql * 8 + xcd;
   const int u_lo = q * p.UQ;
   const int u_hi = min(u_lo + p.UQ, p.U);
-  int lo = (int)p.seg_ptr[F], hi = (int)p.seg_ptr[F + 1];
-  {
-    int a = lo, b = hi;
-    while (a < b) {
-      int mid = (a + b) >> 1;
-      if (p.seg_unit[mid] < u_lo) a = mid + 1; else b = mid;
-    }
-    lo = a;
-    b = hi;
-    while (a < b) {
-      int mid = (a + b) >> 1;
-      if (p.seg_unit[mid] < u_hi) a = mid + 1; else b = mid;
-    }
-    hi = a;
-  }
+  const DxSegs sg = dx_segs(p.seg_ptr, p.seg_unit, p.seg_begin, F, u_lo, u_hi);
   float acc[NS][FW][T];
 #pragma unroll
   for (int sl = 0; sl < NS; ++sl)
@@ -985,14 +917,14 @@ dx_dma_kernel(DxK p) {
 #pragma unroll
     for (int j = 0; j < T; ++j) st.lut[lane][j] = (lane >> j) & 1 ? 1.0f : 0.0f;
   }
-  if (lo < hi) {
-    DxChunk cc{lo, p.seg_begin[lo], p.seg_begin[lo + 1], p.seg_unit[lo]};
+  if (sg.n > 0) {
+    DxChunk cc = dx_first(sg);
     unsigned pe = 0u, pu = 0u;
-    dx_seg_ahead(p, lo, hi, pe, pu);
+    dx_seg_ahead(sg, 0, pe, pu);
     DxChunk cn = cc;
-    dx_next_ahead(p, cn, hi, pe, pu);
+    dx_next_ahead(sg, cn, pe, pu);
     const unsigned rc0 = dx_load_rec(p, cc, lane);
-    unsigned rn = cn.si < hi ? dx_load_rec(p, cn, lane) : 0u;
+    unsigned rn = cn.si < sg.n ? dx_load_rec(p, cn, lane) : 0u;
     dx_dma<K, NS, FLAT>(p, tc0, cc, rc0, st, 0);
     unsigned rc = rc0;
     float c1[NS][T];
@@ -1002,7 +934,7 @@ dx_dma_kernel(DxK p) {
       // every copy, load and LDS read so far is done: buffer cur holds chunk cc, and buffer
       // cur ^ 1 (read by the previous chunk) may be refilled
       __builtin_amdgcn_s_waitcnt(0);
-      const bool more = cn.si < hi;
+      const bool more = cn.si < sg.n;
       float c1n[NS][T];
 #pragma unroll
       for (int sl = 0; sl < NS; ++sl)
@@ -1013,8 +945,8 @@ dx_dma_kernel(DxK p) {
       if (more) {
         // the segment table before the copy: a wait for those loads after it would also wait for
         // the copy (the counter is in order); their values were loaded one step ago
-        dx_next_ahead(p, cnn, hi, pe, pu);
-        if (cnn.si < hi) rnn = dx_load_rec(p, cnn, lane);
+        dx_next_ahead(sg, cnn, pe, pu);
+        if (cnn.si < sg.n) rnn = dx_load_rec(p, cnn, lane);
         dx_dma<K, NS, FLAT>(p, tc0, cn, rn, st, cur ^ 1);
         if (cn.si != cc.si) dx_load_c1_u<NS, FLAT>(p, cn.u, tc0 * 64 * T, lane, c1n);
       }
@@ -1437,21 +1369,7 @@ __global__ void __launch_bounds__(64) dx_dense_kernel(DxK p, const float* __rest
   const int q = ql * 8 + xcd;                        // the pass's partial slot
   const int u_lo = ((p.ql0 + ql) * 8 + xcd) * p.UQ;  // the layer's unit range (p.ql0 + ql) * 8 + xcd
   const int u_hi = min(u_lo + p.UQ, p.U);
-  int lo = (int)p.seg_ptr[F], hi = (int)p.seg_ptr[F + 1];
-  {
-    int a = lo, b = hi;
-    while (a < b) {
-      int mid = (a + b) >> 1;
-      if (p.seg_unit[mid] < u_lo) a = mid + 1; else b = mid;
-    }
-    lo = a;
-    b = hi;
-    while (a < b) {
-      int mid = (a + b) >> 1;
-      if (p.seg_unit[mid] < u_hi) a = mid + 1; else b = mid;
-    }
-    hi = a;
-  }
+  const DxSegs sg = dx_segs(p.seg_ptr, p.seg_unit, p.seg_begin, F, u_lo, u_hi);
   const int tok0 = tc * 64 * T + T * lane;
   float acc[FW][T];
 #pragma unroll
@@ -1467,10 +1385,10 @@ __global__ void __launch_bounds__(64) dx_dense_kernel(DxK p, const float* __rest
   // edges whose rows are in flight together, in two alternating batches (T = 4: 12.6M neurons, 256
   // tokens, 4096 inputs 10.6 ms with 2, 11.4 with 4, 11.4 held to 96 VGPRs for a fifth wave)
   constexpr int DB = T == 4 ? 2 : (T == 2 ? 4 : 8);
-  if (lo < hi) {
-    DxChunk cc{lo, p.seg_begin[lo], p.seg_begin[lo + 1], p.seg_unit[lo]};
+  if (sg.n > 0) {
+    DxChunk cc = dx_first(sg);
     unsigned pe = 0u, pu = 0u;
-    dx_seg_ahead(p, lo, hi, pe, pu);
+    dx_seg_ahead(sg, 0, pe, pu);
     unsigned rec = dx_load_rec(p, cc, lane);
     for (;;) {
       const int n = (int)min(cc.end - cc.e, 64u);
@@ -1526,8 +1444,8 @@ __global__ void __launch_bounds__(64) dx_dense_kernel(DxK p, const float* __rest
       // the next chunk's records land while this chunk is added; the segment table is read a chunk
       // ahead, so nothing here waits behind the rows just requested
       DxChunk cn = cc;
-      dx_next_ahead(p, cn, hi, pe, pu);
-      const bool more = cn.si < hi;
+      dx_next_ahead(sg, cn, pe, pu);
+      const bool more = cn.si < sg.n;
       const unsigned rn = more ? dx_load_rec(p, cn, lane) : 0u;
       for (int i0 = 0; i0 < n; i0 += 2 * DB) {
         load(i0 + DB, vb);

@@ -26,6 +26,9 @@ constexpr unsigned REC_NEWF = 1u << 31;
 // largest token chunk of one backward pass (bounds the per-neuron mask record)
 constexpr int BWD_TOKEN_CHUNK = 1024;
 
+// largest layer, in slots of all pools (check_layer)
+constexpr long long MAX_SLOTS = (1LL << 31) / 16;
+
 constexpr int ceil_div(long long a, long long b) { return (int)((a + b - 1) / b); }
 
 // ---- gather schedule of the neuron-stationary kernels (gl_sched.hip) --------------------------
@@ -174,6 +177,8 @@ __device__ __forceinline__ int opaque(int v) {
   asm volatile("" : "+v"(v));
   return v;
 }
+// a value equal in every lane of the wave, in a scalar register
+__device__ __forceinline__ unsigned wave_uniform(unsigned v) { return (unsigned)__builtin_amdgcn_readfirstlane((int)v); }
 
 // ---- X token tiles: global -> LDS directly ----------------------------------------------------
 // A tile is D float4 slots (4 tokens per input feature).  Every lane copies 16-byte slots with

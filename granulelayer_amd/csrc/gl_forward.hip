@@ -1424,7 +1424,7 @@ int check_layer(int B, int D, int G, int S, int K, int act, int pool, const void
   if (act != GL_ACT_IDENTITY && act != GL_ACT_RELU && act != GL_ACT_GELU) return GL_ERR_UNSUPPORTED;
   if (pool < GL_POOL_MEAN || pool > GL_POOL_SOFTMAX) return GL_ERR_UNSUPPORTED;
   if (x_dtype != GL_DTYPE_F32 && x_dtype != GL_DTYPE_BF16) return GL_ERR_UNSUPPORTED;
-  if ((long long)G * S > (1LL << 31) / 16) return GL_ERR_UNSUPPORTED;
+  if ((long long)G * S > MAX_SLOTS) return GL_ERR_UNSUPPORTED;
   if (D > GL_MAX_INPUTS) return GL_ERR_UNSUPPORTED;  // wider tiles gather from global memory (XG kernels)
   return 0;
 }

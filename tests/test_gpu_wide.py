@@ -212,3 +212,43 @@ def test_bf16_tiles_give_the_bits_of_fp32_tiles():
     counts = L.counts_tensor("cpu").numpy()
     want, mag = O.forward(x.float().numpy(), fi, fw, fb, counts, L.slots_per_group, "relu", "mean", with_mag=True)
     assert_parity(outs[0][0].numpy(), want, mag, what="pre")
+
+
+def test_dx_of_a_layer_with_more_than_2_30_segments():
+    """2^27 neurons of fan-in 16 over 65,536 inputs: 1.36e9 (feature range, unit) segments, more than a
+    32-bit byte offset reaches.  dX of both kernels that read the segment table ahead (masks at 129
+    tokens, per-neuron dz at 2) for dY in 12 pools, the last ones among them."""
+    from granulelayer_amd.layout import SparseLayout
+
+    D, S, G, K = 65536, 512, 262144, 16
+    if torch.cuda.mem_get_info()[0] + torch.cuda.memory_reserved() < 140 * 2**30:
+        pytest.skip("needs 140 GiB of GPU memory")
+    torch.cuda.empty_cache()
+    L = SparseLayout(D, G * S, G, K, 8, False)
+    gen = torch.Generator(device=DEV).manual_seed(0)
+    idx = torch.empty(L.index_shape, dtype=torch.int32, device=DEV).random_(0, D, generator=gen)
+    w = torch.empty(L.weight_shape, device=DEV).uniform_(-0.4, 0.4, generator=gen)
+    b = torch.zeros(L.bias_shape, device=DEV)
+    pools = np.sort(np.concatenate([[0, G - 2, G - 1], np.random.default_rng(0).choice(G - 3, 9, replace=False) + 1]))
+    sel = torch.from_numpy(pools).to(DEV)
+    rows = lambda t: t.view(G, S, -1)[sel].cpu().numpy()  # noqa: E731
+    fi, fw, fb = rows(idx).reshape(-1, K), rows(w).reshape(-1, K), rows(b).reshape(-1)
+    counts = np.full(len(pools), S, np.int32)
+    dw, db = torch.zeros(L.weight_shape, device=DEV), torch.zeros(L.bias_shape, device=DEV)
+    edges = None
+    for B, act in ((129, "relu"), (2, "gelu")):
+        rt = _rt(L, idx, LevelSpec("sum", activation=act))
+        if edges is not None:
+            rt._hip_edges = edges  # the same index tensor
+        x = torch.randn(B, D, generator=gen, device=DEV)
+        dy = torch.zeros(B, G, device=DEV)
+        dy[:, sel] = torch.randn(B, len(pools), generator=gen, device=DEV)
+        dx = rt.backward(x, w, b, dy, {}, "minimal_stats", dw, db).cpu().numpy()
+        edges = rt._hip_edges
+        nseg = int(edges[1][:64].cpu().numpy().view(np.uint32)[10])
+        _, _, dX, bnd = O.backward(x.cpu().numpy(), fi, fw, fb, counts, S, dy[:, sel].cpu().numpy(), act, "sum",
+                                   with_bounds=True)
+        assert_parity(dx, dX, bnd["mag"][2], bnd["unc"][2], what=f"dX ({act})")
+    assert nseg > 2**30
+    del rt, edges, idx, w, dw, x, dy
+    torch.cuda.empty_cache()
