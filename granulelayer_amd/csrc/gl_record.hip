@@ -80,6 +80,13 @@ __device__ __forceinline__ uint4 rec_transpose(uint4 v) {
   const auto d = __builtin_amdgcn_permlane16_swap(a[1], b[1], false, false);
   return make_uint4(c[0], c[1], d[0], d[1]);
 }
+// Orders the wave's LDS accesses on either side, in the compiler as the hardware does by itself: lanes
+// exchange data through LDS that only their own wave touches, so no s_barrier is needed.
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
 // the lane's weights of neuron m (w: its row + 4 G), zero for a padded slot
 __device__ __forceinline__ float4 rec_weights(const float* w, bool valid) {
   uint4 v = *reinterpret_cast<const uint4*>(w);
@@ -246,6 +253,7 @@ __global__ void __launch_bounds__(REC_WAVES * 64, 2) rec_bwd_w_kernel(RecBwdK p)
       if (r >= c.nrec) return;
 #pragma unroll
       for (int j = 0; j < 4; ++j) *reinterpret_cast<float4*>(&xl[(4 * j + G) * REC_XROW + 4 * m]) = xc[j];
+      wave_lds_fence();  // the reads below take rows that other lanes wrote
       if constexpr (r + 1 < REC_PER_WAVE) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) xn[j] = ld_row(xr, off[r + 1][j]);
@@ -263,6 +271,7 @@ __global__ void __launch_bounds__(REC_WAVES * 64, 2) rec_bwd_w_kernel(RecBwdK p)
       float4 xt[4];
 #pragma unroll
       for (int q = 0; q < 4; ++q) xt[q] = *reinterpret_cast<const float4*>(&xl[m * REC_XROW + 16 * G + 4 * q]);
+      wave_lds_fence();  // the next record's rows overwrite them
       float dz[4][4], ds = 0.f;  // [q][i]
 #pragma unroll
       for (int q = 3; q >= 0; --q)
