@@ -93,8 +93,10 @@ def dact_torch(x: torch.Tensor, name: str) -> torch.Tensor:
 
 
 def _g_pre(dy: torch.Tensor, pre: torch.Tensor, name: str) -> torch.Tensor:
-    """dL/dpre = dy * act'(pre); an identity out-activation's factor of 1 needs no launches."""
-    return dy.float() if name == "identity" else dy.float() * dact_torch(pre, name)
+    """dL/dpre = dy * act'(pre); an identity out-activation's factor of 1 needs no launches.  dy may be a
+    lazily negated view (of a conjugate's imaginary part, say), whose memory the kernels would read
+    with the wrong sign."""
+    return dy.float().resolve_neg() if name == "identity" else dy.float() * dact_torch(pre, name)
 
 
 @dataclass

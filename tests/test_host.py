@@ -1,6 +1,7 @@
 """Host logic on the CPU: layout partition, parameter initialisation, configuration parsing,
 refusal of configurations outside the MI355X path, and the synthetic BASELINE generators.
 Mirrors the reference's host-only tests (tests/test_sparse_projection.py:14-51)."""
+import ctypes
 import math
 
 import numpy as np
@@ -122,6 +123,55 @@ def test_runtime_refuses_triton_plan():
     idx, _, _ = init_parameters(L, "cpu")
     with pytest.raises(NotImplementedError, match="Triton"):
         Level1Runtime(L, idx, LevelSpec("mean"), PhysicalPlan(backend="triton"))
+
+
+class _Recorder:
+    """A backend that keeps what the kernels would read at g_pre's address."""
+
+    def __init__(self, layout):
+        self.G, self.read = layout.groups, []
+
+    def forward(self, rt, x, w, b, track_ids=False):
+        pre = torch.zeros(x.shape[0], self.G)
+        return {"pre": pre, "winner": torch.zeros(x.shape[0], self.G, dtype=torch.int32)}
+
+    def backward(self, rt, x, w, b, g_pre, stats, dw_buf, db_buf):
+        assert g_pre.dtype == torch.float32 and g_pre.is_contiguous()
+        raw = (ctypes.c_float * g_pre.numel()).from_address(g_pre.data_ptr())
+        self.read.append(np.array(raw, np.float32).reshape(g_pre.shape))
+        return torch.zeros_like(x)
+
+
+# gradients as autograd hands them over: lazily negated (dense; the imaginary part of a conjugate; one
+# element, where that is contiguous), expanded, transposed, at an odd offset
+DY_VIEWS = {
+    "negated": lambda B, G: torch._neg_view(torch.randn(B, G)),
+    "conj imag": lambda B, G: torch.randn(B, G, dtype=torch.complex64).conj().imag,
+    "expanded": lambda B, G: torch.randn(1, 1).expand(B, G),
+    "transposed": lambda B, G: torch.randn(G, B).t(),
+    "offset": lambda B, G: torch.randn(B * G + 1)[1:].view(B, G),
+}
+
+
+@pytest.mark.parametrize("view", DY_VIEWS)
+@pytest.mark.parametrize("pool,out_act,G,B", [("mean", "identity", 4, 5), ("mean", "identity", 1, 1),
+                                              ("max", "identity", 4, 70), ("mean", "relu", 4, 5)])
+def test_kernels_read_the_values_of_any_gradient_view(monkeypatch, view, pool, out_act, G, B):
+    from granulelayer_amd import autograd as A
+
+    if pool == "max":  # the ids of 32 tokens at a time are recomputed
+        monkeypatch.setattr(A, "CHECKPOINT_BUDGET", 0)
+    L = SparseLayout(64, 50 * G, G, 8, 8, False)
+    idx, w, b = init_parameters(L, "cpu")
+    be = _Recorder(L)
+    rt = Level1Runtime(L, idx, LevelSpec(pool, out_activation=out_act), PhysicalPlan(), backend=be)
+    torch.manual_seed(0)
+    dy = DY_VIEWS[view](B, G)
+    x = torch.randn(B, 64, requires_grad=True)
+    y = A.SparsePoolFunction.apply(x, w.requires_grad_(True), b.requires_grad_(True), rt, "minimal_stats", torch.float32)
+    y.backward(dy)
+    want = dy.numpy(force=True) if out_act == "identity" else np.zeros((B, G), np.float32)  # relu'(0) = 0
+    assert np.array_equal(np.concatenate(be.read), want)
 
 
 def test_fused_adamw_refuses_what_it_cannot_update():
