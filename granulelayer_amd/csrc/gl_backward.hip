@@ -1799,6 +1799,15 @@ static bool dx_short_segments(const GlBwdArgs* a) {
 static bool bwd_rec_layer(const GlBwdArgs* a) {
   return a->act != GL_ACT_GELU && record_layer(a->K, a->rec_shift, a->pool, a->w_dtype);
 }
+// ... for this chunk of tokens.  Tokens at which both dW passes take the same time (4M neurons in pools
+// of 512): 46 at D = 256, 42 at 1024, 34 at 4096, 33 at 16,384 and 65,536, 30 at 8192 with bf16 X and 23
+// with the two-token tiles of fp32 X; 6 and 16 with pools of 16 and 48 slots.  At D = 4096 the backward
+// per-neuron / record: 4 tokens 1212 / 1393 us, 24 1337 / 1397, 48 1493 / 1400, 64 1593 / 1408.
+static bool bwd_rec(const GlBwdArgs* a, int Bc) {
+  if (!bwd_rec_layer(a) || !record_aligned(a->W, a->bias, a->idx) || ((uintptr_t)a->dW & 15) != 0) return false;
+  const int least = a->D <= XTILE_DB / 2 ? 44 : (tiles_of_two(a->D) && a->x_dtype == GL_DTYPE_F32 ? 23 : 32);
+  return record_pays(Bc, a->S, 64 * bwd_npl(16), least);
+}
 
 extern "C" int gl_bwd_workspace(const GlBwdArgs* a, size_t* bytes) {
   if (!a || !bytes) return GL_ERR_ARG;
@@ -1875,7 +1884,7 @@ extern "C" int gl_bwd(const GlBwdArgs* a, void* stream) {
     // two-token fp32 tiles: half the gathers and tile overheads per token for one widening per value)
     const bool xb = (wide && a->x_dtype == GL_DTYPE_BF16) || (win && xbw);
     const int tb = wide && !xb ? 2 : BT;
-    const bool rec = bwd_rec_layer(a) && record_aligned(a->W, a->bias, a->idx) && ((uintptr_t)a->dW & 15) == 0;
+    const bool rec = bwd_rec(a, Bc);
     if (rec)
       GL_TRY(launch_slice_x(a->X, a->sxb, a->x_dtype, a->B, a->D, b0, ceil_div(Bc, 64), (float*)xt, s));
     else if (xb)

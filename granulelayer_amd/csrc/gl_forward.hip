@@ -1293,12 +1293,27 @@ static long long fwd_part_per_token(const GlFwdArgs* a, long long n_chunks) {
   return n_chunks * kp * 4 * (sel ? 2 : 1);
 }
 
-static bool fwd_rec(const GlFwdArgs* a) {
-  return record_layer(a->K, a->rec_shift, a->pool, a->w_dtype) && record_aligned(a->W, a->bias, a->idx);
+// The record kernels run this call, passes of `tokens` tokens.  Tokens at which they and the per-neuron
+// kernels take the same time (4M neurons in pools of 512, fp32 X): ReLU 32 at D = 256, 29 at 1024, 20 at
+// 4096, 16 at 8192, 14 at 16,384, 16 at 65,536; GELU (bound by its 16 erf per lane and slice) 26, 24,
+// 20, 32, 33, 33, and with bf16 X, whose per-neuron tiles run two workgroups per CU, 43 at 4096 and 38
+// at 8192; staged pool windows of wider layers run as D <= 4096 does (GELU, 32 tokens 525 / 365 us).  At
+// D = 4096 per-neuron / record: ReLU 4 tokens 80 / 151 us, 16 135 / 152, 24 170 / 153, 64 351 / 158;
+// GELU 131 / 316, 301 / 354, 414 / 360, 980 / 366.  Pools of 128 slots: 16 tokens 109 / 74.
+static bool fwd_rec(const GlFwdArgs* a, long long tokens) {
+  if (!record_layer(a->K, a->rec_shift, a->pool, a->w_dtype) || !record_aligned(a->W, a->bias, a->idx)) return false;
+  const bool xb = a->x_dtype == GL_DTYPE_BF16 && a->D % 2 == 0 && a->D <= 2 * XTILE_DB;
+  int ww, npw;
+  const bool lds_f32 = !xb && (a->D <= XTILE_DB ||
+                               window_staging(a->win, a->win_width, a->D, fwd_waves(16, PK_SUM, a->act),
+                                              ceil_div(a->S, 64 * FWD_NPL), a->G, &ww, &npw));
+  const int least = a->act == GL_ACT_GELU ? (lds_f32 ? 20 : 36) : (a->D <= XTILE_DB / 2 ? 28 : 16);
+  return record_pays(tokens, a->S, 64 * FWD_NPL, least);
 }
 
 // plan with token chunks of at most bf_cap tokens (<= 0: no cap beyond the part budget)
-// rec: with the record kernels (fwd_rec)
+// rec: with the record kernels (fwd_rec); chosen by the whole batch, so that any part budget gives the
+// same bits
 static FwdPlan fwd_plan(const GlFwdArgs* a, bool rec, long long bf_cap = 0) {
   FwdPlan q;
   q.rec = rec;
@@ -1597,7 +1612,8 @@ static int fwd_run(const GlFwdArgs* a, void* ws, const FwdPlan& q, hipStream_t s
 // copy per GPU, held until the process ends) instead of a caller workspace, for callers that cannot
 // allocate.  Host code never passes the array's name to a kernel: it passes the per-device address
 // that hipGetSymbolAddress returns.  The forward runs as many token passes as the array needs; the
-// results are those of gl_fwd (every token's arithmetic and order are the same).
+// results are those of gl_fwd (every token's arithmetic and order are the same; layers of shared records
+// too large for whole passes may sum in another order, gl_fwd_static).
 static __device__ __align__(256) unsigned char scratch[GL_FWD_STATIC_SCRATCH_BYTES];
 
 namespace {
@@ -1680,7 +1696,7 @@ extern "C" int gl_fwd(const GlFwdArgs* a, void* stream) {
   GL_TRY(gl_fwd_workspace(a, &need));
   if (!a->ws || a->ws_bytes < need) return GL_ERR_WORKSPACE;
   if (a->sched && a->K != 8) return GL_ERR_UNSUPPORTED;
-  return fwd_run(a, a->ws, fwd_plan(a, fwd_rec(a)), (hipStream_t)stream);
+  return fwd_run(a, a->ws, fwd_plan(a, fwd_rec(a, a->B)), (hipStream_t)stream);
 }
 
 extern "C" int gl_fwd_static(const GlFwdArgs* a, void* stream) {
@@ -1689,10 +1705,13 @@ extern "C" int gl_fwd_static(const GlFwdArgs* a, void* stream) {
   size_t need = 0;
   GL_TRY(gl_fwd_workspace(a, &need));  // argument checks; ws / ws_bytes are ignored
   if (a->sched && a->K != 8) return GL_ERR_UNSUPPORTED;
-  // a record layer whose 128-slot partials do not fit runs the per-neuron kernels (256-slot partials)
-  bool rec = fwd_rec(a);
+  // The record kernels' 128-slot partials leave room for half the tokens of the per-neuron kernels'
+  // 256-slot ones.  Where that makes their passes short (fewer than 24 tokens with ReLU at D = 4096, for
+  // layers of more than 80M neurons) the per-neuron kernels are faster, and their sums are those of
+  // another order.
+  bool rec = fwd_rec(a, a->B);
   long long bf = static_chunk(a, rec);
-  if (rec && bf < BT) rec = false, bf = static_chunk(a, false);
+  if (rec && bf < a->B && !fwd_rec(a, bf * 2 / 3)) rec = false, bf = static_chunk(a, false);
   if (bf < BT) return GL_ERR_SCRATCH;
   const FwdPlan q = fwd_plan(a, rec, bf);
   if (q.xt_bytes + q.part_bytes + q.slot_bytes > (size_t)GL_FWD_STATIC_SCRATCH_BYTES) return GL_ERR_SCRATCH;

@@ -90,11 +90,18 @@ int launch_max_events(int K, int act, const MaxEvKArgs& a, hipStream_t s);
 // 16 x 16 products on the matrix cores.  X goes through slices of 64 tokens ([slice][D][64] fp32), a
 // wave takes REC_CHUNK slots.  record_layer: the layer qualifies (workspaces are sized by it alone,
 // whatever the pointers); record_aligned: these pointers do too.  Other layers with shared records
-// (other shifts, fan-in 8, bf16 parameters, views off a 16-byte boundary) run the per-neuron kernels.
+// (other shifts, fan-in 8, bf16 parameters, views off a 16-byte boundary) and calls of few tokens
+// (record_pays) run the per-neuron kernels.
 constexpr int REC_CHUNK = 128;
 bool record_layer(int K, int rec_shift, int pool, int w_dtype);
 inline bool record_aligned(const void* a, const void* b, const void* c) {
   return (((uintptr_t)a | (uintptr_t)b | (uintptr_t)c) & 15) == 0;
+}
+// A slice of 64 tokens costs a record the same however few of them are real, and a per-neuron chunk of
+// `chunk` slots the same however few the pool fills: the record kernels pay from `least` tokens on, less
+// by the share of a chunk that a pool of S slots leaves empty.
+inline bool record_pays(long long tokens, int S, int chunk, int least) {
+  return tokens * round_up(S, chunk) > (long long)least * S;
 }
 int launch_slice_x(const void* X, long long sxb, int x_dtype, int B, int D, int b0, int n_slices, float* xs,
                    hipStream_t s);

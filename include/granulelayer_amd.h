@@ -243,8 +243,9 @@ int gl_fwd_mask_bytes(const GlFwdArgs* a, size_t* bytes);
  * loops, harnesses that forbid hipMalloc).  The token tiles and partial results live in a
  * library-owned static device array of GL_FWD_STATIC_SCRATCH_BYTES per GPU (held from the first
  * call on that GPU until the process ends); a->ws, a->ws_bytes are ignored.  The forward runs as
- * many token passes as the array needs, with the results of gl_fwd; layers whose partials for one
- * 4-token tile exceed the array are refused with GL_ERR_SCRATCH.  Every call on a GPU shares that
+ * many token passes as the array needs, with the results of gl_fwd (bit for bit, but for layers with
+ * rec_shift 4 of more than about 80M slots: their sums may run in another order); layers whose
+ * partials for one 4-token tile exceed the array are refused with GL_ERR_SCRATCH.  Every call on a GPU shares that
  * GPU's array.  Outside graph capture, calls on different streams of one GPU are ordered by a
  * per-device "last use" event (each call's launches wait for the previous call's); under graph
  * capture the caller's graph must order the calls that share a GPU, or they race.  Nothing in it

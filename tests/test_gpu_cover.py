@@ -310,3 +310,92 @@ def test_record_forward_in_token_passes_and_without_a_workspace():
     assert N.library().lib.gl_fwd_static(ctypes.byref(a), ctypes.c_void_p(_stream(x.device))) == 0
     for o in (*outs[1:], pre):
         assert torch.equal(o, outs[0])
+
+
+def _off_boundary(t):
+    """A copy of t that starts 4 bytes past a 16-byte boundary: the per-neuron kernels take it."""
+    return torch.empty(t.numel() + 1, device=t.device, dtype=t.dtype)[1:].view(t.shape).copy_(t)
+
+
+# (act, D, neurons per pool, x dtype, tokens of the last per-neuron call, of the first record call): the
+# record kernels pay from 28 (16 past 2048 inputs) tokens with ReLU and 20 (36) with GELU, times the share
+# of a 256-slot chunk that the pool fills
+@pytest.mark.parametrize("act,D,per,xdt,last,first", [
+    ("relu", 64, 256, torch.float32, 28, 29),
+    ("relu", 2049, 256, torch.float32, 16, 17),
+    ("relu", 64, 520, torch.float32, 19, 20),       # 528 slots in 3 chunks of 256
+    ("identity", 64, 16, torch.float32, 1, 2),
+    ("gelu", 64, 1000, torch.float32, 19, 20),      # 1008 slots in 4 chunks
+    ("gelu", 64, 256, torch.bfloat16, 36, 37),
+])
+def test_record_forward_from_the_tokens_it_pays_at(act, D, per, xdt, last, first):
+    """Fewer tokens give the per-neuron kernels' sums bit for bit, more another order of the same terms."""
+    from granulelayer_amd import LevelSpec, PhysicalPlan
+    from granulelayer_amd.autograd import Level1Runtime
+
+    lay = _record_layer(D, per, 64)
+    rt = Level1Runtime(lay.layout, lay.indices, LevelSpec("sum", activation=act), PhysicalPlan())
+    w = lay.weight.detach()
+    x = torch.randn(first, D, device=DEV).to(xdt)
+    for B, rec in ((last, False), (first, True)):
+        pre, per_neuron = (rt.forward(x[:B], v, lay.bias)["pre"] for v in (w, _off_boundary(w)))
+        assert torch.equal(pre, per_neuron) != rec
+        assert_close(pre.cpu().numpy(), per_neuron.cpu().numpy(), rtol=1e-5, atol=1e-5 * per ** 0.5)
+
+
+@pytest.mark.parametrize("D,per,last,first", [(64, 512, 44, 45), (2050, 512, 32, 33), (64, 48, 16, 17)])
+def test_record_dw_from_the_tokens_it_pays_at(D, per, last, first):
+    """As above for the dW pass; a batch's last chunk of 1024 tokens decides for itself."""
+    from granulelayer_amd import LevelSpec, PhysicalPlan
+    from granulelayer_amd.autograd import Level1Runtime
+
+    lay = _record_layer(D, per, 64)
+    rt = Level1Runtime(lay.layout, lay.indices, LevelSpec("sum", activation="relu"), PhysicalPlan())
+    w = lay.weight.detach()
+    x, dy = torch.randn(first, D, device=DEV), torch.randn(first, 64, device=DEV)
+    for B, rec in ((last, False), (first, True)):
+        out = []
+        for v in (w, _off_boundary(w)):
+            dw, db = torch.zeros_like(w), torch.zeros_like(lay.bias)
+            dx = rt.backward(x[:B], v, lay.bias, dy[:B], {}, "minimal_stats", dw, db)
+            out.append((dw, db, dx))
+        assert torch.equal(out[0][0], out[1][0]) != rec
+        assert torch.equal(out[0][2], out[1][2])  # the same mask bits
+        for a, b in zip(*out):
+            assert_close(a.detach().cpu().numpy(), b.detach().cpu().numpy(), rtol=1e-5, atol=2e-5)
+
+
+@pytest.mark.parametrize("per,pools,rec", [(16, 400_000, True), (256, 330_000, False)])
+def test_static_forward_of_record_layers_in_short_passes(per, pools, rec):
+    """gl_fwd_static where fewer than 64 tokens' partials fit its scratch: passes of 36 tokens on the record
+    kernels give gl_fwd's bits; where 128-slot partials leave 20 tokens a pass, the per-neuron kernels
+    (256-slot partials) give their own."""
+    import ctypes
+
+    from granulelayer_amd import LevelSpec, PhysicalPlan
+    from granulelayer_amd import _native as N
+    from granulelayer_amd.autograd import Level1Runtime
+    from granulelayer_amd.backend import _ptr, _stream
+
+    D, B = 64, 70
+    lay = CoverTopK16Layer(D, pools * per, pools, per, pooling="mean", device=DEV)
+    L = lay.layout
+    gen = torch.Generator(device=DEV).manual_seed(0)
+    with torch.no_grad():
+        lay.indices.random_(0, D, generator=gen)
+        lay.weight.normal_(0, 0.25, generator=gen)
+        lay.bias.normal_(0, 0.25, generator=gen)
+    x = torch.randn(B, D, device=DEV, generator=gen)
+    rt = Level1Runtime(L, lay.indices, LevelSpec("sum", activation="relu"), PhysicalPlan())
+    w = lay.weight.detach()
+    pre = torch.empty(B, pools, device=DEV)
+    a = N.GlFwdArgs(X=_ptr(x), sxb=D, x_dtype=N.GL_DTYPE_F32, B=B, D=D, G=pools, S=per, K=16, act=N.GL_ACT["relu"],
+                    pool=N.GL_POOL["sum"], rec_shift=4, idx=_ptr(lay.indices), W=_ptr(w), bias=_ptr(lay.bias),
+                    counts=_ptr(rt.counts_i32), pre=_ptr(pre))
+    assert N.library().lib.gl_fwd_static(ctypes.byref(a), ctypes.c_void_p(_stream(x.device))) == 0
+    full = rt.forward(x, w, lay.bias)["pre"]
+    per_neuron = rt.forward(x, _off_boundary(w), lay.bias)["pre"]
+    assert torch.equal(pre, full if rec else per_neuron)
+    assert torch.equal(full, per_neuron) is False
+    err = (full - per_neuron).abs()
+    assert bool((err <= 1e-5 * per_neuron.abs() + 1e-5 * per ** 0.5).all())
