@@ -236,6 +236,11 @@ def _record_layer(D, per, G, seed=0):
     return lay
 
 
+def _off_boundary(t):
+    """A copy of t that starts 4 bytes past a 16-byte boundary: the per-neuron kernels take it."""
+    return torch.empty(t.numel() + 1, device=t.device, dtype=t.dtype)[1:].view(t.shape).copy_(t)
+
+
 @pytest.mark.parametrize("act,pool", [("relu", "sum"), ("identity", "mean"), ("gelu", "sum")])
 @pytest.mark.parametrize("case", RECORD_CASES, ids=lambda c: f"D{c[0]}n{c[1]}B{c[3]}{str(c[4])[6:]}")
 def test_record_kernels_match_oracle(case, act, pool):
@@ -267,10 +272,17 @@ def test_record_kernels_match_oracle(case, act, pool):
     valid = L.valid_mask("cpu").reshape(-1).numpy()
     assert not dw.cpu().numpy().reshape(-1, 16)[~valid].any() and not db.cpu().numpy().reshape(-1)[~valid].any()
     # views off a 16-byte boundary run the per-neuron kernels: the same z bit for bit (pools of one
-    # slot show them), the same sums in another order
-    off = torch.empty(lay.weight.numel() + 1, device=DEV)[1:].view(lay.weight.shape).copy_(lay.weight.detach())
+    # slot show them), the same sums in another order; the backward also with an unaligned dW
+    off = _off_boundary(lay.weight.detach())
     pre = rt.forward(xd, off, lay.bias)["pre"].cpu().numpy()
     assert_parity(pre, want, mag, what="pre (unaligned weights)")
+    for wv, dw in ((off, torch.zeros(L.weight_shape, device=DEV)),
+                   (lay.weight.detach(), _off_boundary(torch.zeros(L.weight_shape, device=DEV)))):
+        db = torch.zeros(L.bias_shape, device=DEV)
+        dx = rt.backward(xd, wv, lay.bias, dy.to(DEV), {"pre": got["pre"]}, "minimal_stats", dw, db)
+        assert_parity(dw.cpu().numpy().reshape(-1, 16), dW, mW, uW, what="dW (unaligned)")
+        assert_parity(db.cpu().numpy().reshape(-1), dB, mb, ub, what="db (unaligned)")
+        assert_parity(dx.cpu().numpy(), dX, mX, uX, what="dX (unaligned)")
 
 
 def test_record_z_has_the_bits_of_the_per_neuron_kernels():
@@ -310,11 +322,6 @@ def test_record_forward_in_token_passes_and_without_a_workspace():
     assert N.library().lib.gl_fwd_static(ctypes.byref(a), ctypes.c_void_p(_stream(x.device))) == 0
     for o in (*outs[1:], pre):
         assert torch.equal(o, outs[0])
-
-
-def _off_boundary(t):
-    """A copy of t that starts 4 bytes past a 16-byte boundary: the per-neuron kernels take it."""
-    return torch.empty(t.numel() + 1, device=t.device, dtype=t.dtype)[1:].view(t.shape).copy_(t)
 
 
 # (act, D, neurons per pool, x dtype, tokens of the last per-neuron call, of the first record call): the
@@ -399,3 +406,30 @@ def test_static_forward_of_record_layers_in_short_passes(per, pools, rec):
     assert torch.equal(full, per_neuron) is False
     err = (full - per_neuron).abs()
     assert bool((err <= 1e-5 * per_neuron.abs() + 1e-5 * per ** 0.5).all())
+
+
+@pytest.mark.parametrize("act", ["relu", "identity"])
+def test_record_kernels_pass_infinities_and_nan_like_the_per_neuron_kernels(act):
+    """X with infinities and NaN: the same outputs and gradients are infinite or NaN (the tokens beside the
+    bad ones stay out of it), the others agree.  Input 0 stays finite: the per-neuron kernels' padded
+    slots read it with weight 0."""
+    from granulelayer_amd import LevelSpec, PhysicalPlan
+    from granulelayer_amd.autograd import Level1Runtime
+
+    D, B, G = 40, 100, 6
+    lay = _record_layer(D, 37, G)  # a partial record: 11 padded slots with weights of their own
+    x, dy = torch.randn(B, D, device=DEV), torch.randn(B, G, device=DEV)
+    x[3, 5], x[64, 1], x[99, 7] = float("inf"), float("nan"), -float("inf")
+    rt = Level1Runtime(lay.layout, lay.indices, LevelSpec("sum", activation=act), PhysicalPlan())
+    out = []
+    for w in (lay.weight.detach(), _off_boundary(lay.weight.detach())):
+        pre = rt.forward(x, w, lay.bias)["pre"]
+        dw, db = torch.zeros(lay.layout.weight_shape, device=DEV), torch.zeros(lay.layout.bias_shape, device=DEV)
+        dx = rt.backward(x, w, lay.bias, dy, {}, "minimal_stats", dw, db)
+        out.append((pre.detach(), dw, db, dx))
+    for a, b in zip(*out):
+        fin = torch.isfinite(a)
+        assert torch.equal(fin, torch.isfinite(b)) and torch.equal(a.isnan(), b.isnan()) and bool(fin.any())
+        assert torch.equal(a[a.isinf()], b[b.isinf()])
+        assert_close(a[fin].cpu().numpy(), b[fin].cpu().numpy(), rtol=1e-5, atol=5e-5)
+    assert not bool(torch.isfinite(out[0][0]).all()) and not bool(torch.isfinite(out[0][1]).all())

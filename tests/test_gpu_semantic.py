@@ -187,8 +187,9 @@ def test_max_of_shard_maxima_is_the_flat_maximum_on_the_gpu():
 def test_shard_dx_equals_the_plain_pools(full, K, B):
     """Shards that fill their groups lie back to back like plain pools of their size (the dX kernels'
     flat units): dX, dW and db of the same neurons as 4 shards per group and as 4 G pools agree bit for
-    bit.  With a last shard that ends inside the group the units take the general form; the same pools
-    exist as plain layout pools of unequal size only, so there the oracle's bar on dX applies."""
+    bit.  With a last shard that ends inside the group the units take the general form: its neurons
+    laid out as full shards whose counts end the same way (flat units) give the same bits.  Both against
+    the oracle."""
     G, nps, D = 6, 64, 200
     per = 4 * nps if full else 4 * nps - 32
     L = SparseLayout(D, G * per, G, K, 8, False)
@@ -196,22 +197,34 @@ def test_shard_dx_equals_the_plain_pools(full, K, B):
     gen = torch.Generator().manual_seed(B)
     x, dy = torch.randn(B, D, generator=gen).to(DEV), torch.randn(B, 4 * G, generator=gen)
 
-    def backward(layout, i, wt, bt, nps_):
+    def backward(layout, i, wt, bt, nps_, unit_counts=None):
         rt = Level1Runtime(layout, i.to(DEV), LevelSpec("sum", activation="relu"), PhysicalPlan(), nps_)
+        if unit_counts is not None:
+            rt.unit_counts_i32 = torch.from_numpy(unit_counts).to(DEV)
         dw, db = torch.zeros(layout.weight_shape, device=DEV), torch.zeros(layout.bias_shape, device=DEV)
         dx = rt.backward(x, wt.to(DEV), bt.to(DEV), dy.to(DEV), {}, "minimal_stats", dw, db)
-        return dx, dw.reshape(-1), db.reshape(-1)
+        return dx, dw.reshape(-1, K), db.reshape(-1)
 
     got = backward(L, idx, w, b, nps)
+    # the neurons as pools of nps slots, the last one of a group padded where it is ragged
+    counts = np.array([nps, nps, nps, nps - (4 * nps - per)] * G, np.int32)
+    pad = (0, 0, 0, 4 * nps - per)
+    fi, fw, fb = (torch.nn.functional.pad(t.reshape(G, per, -1), pad).reshape(G * 4 * nps, -1) for t in (idx, w, b))
+    valid = (torch.arange(nps)[None, :] < torch.from_numpy(counts)[:, None]).reshape(-1).to(DEV)
     if full:
         P = SparseLayout(D, G * per, 4 * G, K, 8, False)
         want = backward(P, idx.view(P.index_shape), w.view(P.weight_shape), b.view(P.bias_shape), None)
-        for name, a, c in zip(("dX", "dW", "db"), got, want):
-            assert torch.equal(a, c), name
-        return
-    counts = np.array([nps, nps, nps, nps - 32] * G, np.int32)  # oracle pools of nps slots, the last ones padded
-    fi, fw, fb = (t.reshape(G, per, -1).numpy() for t in (idx, w, b))
-    pad = ((0, 0), (0, 32), (0, 0))
-    fi, fw, fb = (np.pad(t, pad).reshape(G * 4 * nps, -1) for t in (fi, fw, fb))
-    _, _, dX, bnd = O.backward(x.cpu().numpy(), fi, fw, fb[:, 0], counts, nps, dy.numpy(), "relu", "sum", with_bounds=True)
-    assert_parity(got[0].cpu().numpy(), dX, bnd["mag"][2], bnd["unc"][2], what="dX")
+    else:
+        P = SparseLayout(D, G * 4 * nps, G, K, 8, False)
+        want = backward(P, fi.view(P.index_shape), fw.view(P.weight_shape), fb.view(P.bias_shape), nps, counts)
+        assert not want[1][~valid].any() and not want[2][~valid].any()
+    want = (want[0], want[1][valid], want[2][valid])
+    for name, a, c in zip(("dX", "dW", "db"), got, want):
+        assert torch.equal(a, c), name
+    dW, db, dX, bnd = O.backward(x.cpu().numpy(), fi.numpy(), fw.numpy(), fb[:, 0].numpy(), counts, nps, dy.numpy(), "relu",
+                                 "sum", with_bounds=True)
+    v = valid.cpu().numpy()
+    for name, a, c, mag, unc in zip(("dW", "db", "dX"), (got[1], got[2], got[0]), (dW[v], db[v], dX),
+                                    (bnd["mag"][0][v], bnd["mag"][1][v], bnd["mag"][2]),
+                                    (bnd["unc"][0][v], bnd["unc"][1][v], bnd["unc"][2])):
+        assert_parity(a.cpu().numpy(), c, mag, unc, what=name)

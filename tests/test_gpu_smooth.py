@@ -218,10 +218,11 @@ def test_power_mean_integer_p(case, p):
     assert_parity(db.cpu().numpy().reshape(-1), wdb, mb, what=f"p {p} db")
 
 
-# the dense dX at its edges: one feature range (D = 16, 24), segments of one edge to several 64-edge
-# chunks (pools of 9 to 1100 slots), tokens around the 64 / 128 / 256-token slices, bf16 weights
+# the dense dX at its edges: one, two and three feature ranges of 8 (D = 8, 16, 24), segments of one edge to
+# several 64-edge chunks (pools of 9 to 1100 slots), tokens around the 64 / 128 / 256-token slices, bf16 weights
 DENSE_DX_EDGES = [
     # D, H, G, K, B, w dtype
+    (8, 200, 3, 8, 70, torch.float32),
     (16, 9, 1, 8, 1, torch.float32),
     (24, 330, 30, 16, 63, torch.float32),
     (17, 2200, 2, 8, 64, torch.bfloat16),
