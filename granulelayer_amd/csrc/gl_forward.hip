@@ -830,7 +830,11 @@ __global__ void __launch_bounds__(WAVES * 64, SMALL ? (K == 16 && PK != PK_SUM ?
   // (whole tiles staged, p.win null: one window of all inputs)
   const int pk = WS && p.win ? (int)(g - g_first) : 0;
   const int lo = WS && p.win ? (int)__builtin_amdgcn_readfirstlane(p.win[g]) : 0;
-  // the lane's neurons: input addresses, weights, bias, slots
+  // the lane's neurons: input addresses, weights, bias, slots.  A padded slot (weight and bias 0) reads
+  // input 0, whose infinity or NaN then makes identity and GELU pools NaN; at fan-in 16 sum / mean it
+  // reads the inputs of the pool's first slot, so a finite pool stays finite as in the record kernels
+  constexpr bool PAD_FIRST = K == 16 && PK == PK_SUM;
+  const int s_pad = PAD_FIRST ? 0 : ext - 1;
   constexpr bool NARROW = WS && SMALL && PK != PK_SUM;  // whole tiles only (p.win null)
   if constexpr (WS && !NARROW) {
     // pool windows: the parameter dtype tested per load (the set-up below, written as a generic
@@ -840,12 +844,12 @@ __global__ void __launch_bounds__(WAVES * 64, SMALL ? (K == 16 && PK != PK_SUM ?
       uint32_t order;
       const int s = sched_slot(p.sched, p.nwin, p.S, g, s_lo, j, lane, order);
       const bool valid = s < n_g;
-      const long long n = nb + (s < ext ? s : ext - 1);  // in-bounds address; invalid slots masked
+      const long long n = nb + (s < (PAD_FIRST ? n_g : ext) ? s : s_pad);  // in-bounds address; invalid slots masked
 #pragma unroll
       for (int ks = 0; ks < K; ++ks) {
         const int k = sched_k<K>(order, ks);  // the pooled sum does not depend on the visiting order
         int d = rec_index(p.idx, n, k, K, p.rs);
-        d = (d < 0 || !valid) ? 0 : (d >= p.D ? p.D - 1 : d);  // host validates; clamp keeps LDS reads in bounds
+        d = (d < 0 || (!valid && !PAD_FIRST)) ? 0 : (d >= p.D ? p.D - 1 : d);  // host validates; clamp keeps LDS reads in bounds
         addr[j][ks] = win_addr<SLOT>(d, pk, lo, p.ww);
         const float wl = ld_param(p.W, p.wbf, n * K + k);
         w[j][ks] = valid ? wl : 0.f;
@@ -865,12 +869,12 @@ __global__ void __launch_bounds__(WAVES * 64, SMALL ? (K == 16 && PK != PK_SUM ?
         uint32_t order;
         const int s = sched_slot(p.sched, p.nwin, p.S, g, s_lo, j, lane, order);
         const bool valid = s < n_g;
-        const long long n = nb + (s < ext ? s : ext - 1);  // in-bounds address; invalid slots masked
+        const long long n = nb + (s < (PAD_FIRST ? n_g : ext) ? s : s_pad);  // in-bounds address; invalid slots masked
 #pragma unroll
         for (int ks = 0; ks < K; ++ks) {
           const int k = sched_k<K>(order, ks);  // the pooled sum does not depend on the visiting order
           int d = rec_index(p.idx, n, k, K, p.rs);
-          d = (d < 0 || !valid) ? 0 : (d >= p.D ? p.D - 1 : d);  // host validates; clamp keeps LDS reads in bounds
+          d = (d < 0 || (!valid && !PAD_FIRST)) ? 0 : (d >= p.D ? p.D - 1 : d);  // host validates; clamp keeps LDS reads in bounds
           addr[j][ks] = (unsigned)d * SLOT;
           const float wl = ld_param_t<BF>(p.W, n * K + k);
           w[j][ks] = valid ? wl : 0.f;

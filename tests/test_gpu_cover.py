@@ -433,3 +433,26 @@ def test_record_kernels_pass_infinities_and_nan_like_the_per_neuron_kernels(act)
         assert torch.equal(a[a.isinf()], b[b.isinf()])
         assert_close(a[fin].cpu().numpy(), b[fin].cpu().numpy(), rtol=1e-5, atol=5e-5)
     assert not bool(torch.isfinite(out[0][0]).all()) and not bool(torch.isfinite(out[0][1]).all())
+
+
+@pytest.mark.parametrize("act", ["identity", "gelu", "relu"])
+@pytest.mark.parametrize("B", [8, 70])
+def test_padded_slots_keep_finite_pools_finite(act, B):
+    """An infinity or NaN reaches only the pools that have a neuron reading it: padded slots add nothing,
+    in the record kernels and in the per-neuron kernels of few tokens."""
+    from granulelayer_amd import LevelSpec, PhysicalPlan
+    from granulelayer_amd.autograd import Level1Runtime
+
+    D, G, per = 300, 50, 37
+    lay = _record_layer(D, per, G)
+    rt = Level1Runtime(lay.layout, lay.indices, LevelSpec("mean", activation=act), PhysicalPlan())
+    x = torch.randn(B, D, device=DEV)
+    x[2, 0], x[5, 0], x[6, 9] = float("nan"), float("inf"), -float("inf")
+    idx = lay.indices.view(G, -1)  # every record has a valid neuron
+    reads = {d: (idx == d).any(1) for d in (0, 9)}
+    assert 0 < int(reads[0].sum()) < G and 0 < int(reads[9].sum()) < G
+    finite = torch.isfinite(rt.forward(x, lay.weight.detach(), lay.bias)["pre"])
+    assert bool(finite[2][~reads[0]].all()) and bool(finite[5][~reads[0]].all()) and bool(finite[6][~reads[9]].all())
+    assert bool(torch.cat([finite[:2], finite[3:5], finite[7:]]).all())
+    if act == "identity":
+        assert not bool(finite[2][reads[0]].any())
