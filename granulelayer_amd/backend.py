@@ -10,8 +10,8 @@ sparse_pooling/backends/cuda/runtime.py:339-712):
 plus ``adam`` (the FusedAdamW launch, sparse_pooling/optim.py:116-123) and ``edges`` (the
 input-major edge list the deterministic dX kernel consumes, built once per index tensor).
 
-Every launch runs under ``torch.cuda.device(<tensor device>)`` on that device's current stream,
-asynchronously; buffers (outputs and workspace) are allocated by PyTorch and passed as raw
+Every launch runs with the tensors' device current (switched to where it is not, ``_on``), on that
+device's current stream, asynchronously; buffers (outputs and workspace) are allocated by PyTorch and passed as raw
 pointers.  Any refusal of the native library raises ``NativeError``; there is no fallback.
 """
 from __future__ import annotations

@@ -826,9 +826,9 @@ __device__ __forceinline__ void dx_dma(const DxK& p, int tc0, const DxChunk& c, 
   }
 }
 
-// dx_run over the DMA layout, edges i .. i1 - 1: mrow = LDS address of the lane's mask word of edge 0 in
-// slice 0 (rows 16 bytes apart, slice s DX_SLICE_WORDS further); wl = the weight of the lane's own edge, edge i's weight
-// taken from lane i (v_readlane, one VALU instead of one more LDS read per edge)
+// dx_run over the DMA layout, edges i0 .. i1 - 1: mrow = LDS address of the lane's mask word of edge 0
+// in slice 0 (rows 16 bytes apart, slice s DX_SLICE_WORDS further); wl = the weight of the lane's own
+// edge, edge i's weight taken from lane i (v_readlane, one VALU instead of one more LDS read per edge)
 template <int X, int NS>
 __device__ __forceinline__ void dx_run_dma(const unsigned* mrow, float wl, const float (*lut)[4], int i0, int i1,
                                            unsigned bit, const float (&c1)[NS][4], float (&acc)[NS][FW][4]) {
@@ -1350,12 +1350,14 @@ __device__ __forceinline__ void dx_add_run(int f, const float (&r)[T], float (&a
 // Each edge's row offset, weight and feature are computed once, in the edge's own lane, and taken
 // with v_readlane: the row is one buffer load with the unit's resource and the offset as its scalar
 // offset, and a bit mask of the run starts replaces the comparison of features.  Built from scalars
-// per edge, the 64-bit row address, the resource and the comparisons took ~34 scalar instructions, and
-// their issue (one per 4 clocks and SIMD: 136 clocks per edge) bounded the kernel at T = 1 and 2.
+// per edge, the 64-bit row address, the resource and the comparisons made scalar issue (one per 4
+// clocks and SIMD) the bound at T = 1 and 2.  Counted at fan-in 16, 77 tokens: 28 scalar instructions
+// per edge, 0.56 ms of issue in 0.73 ms, now 9.4; at 12.6M neurons, 256 tokens: 33, now 18.
 // Lanes past the chunk's Bc tokens load nothing (their offset is out of the resource's range).
 // LogMeanExp dX before -> now: 4M neurons, 64 tokens, 1024 inputs 1.82 -> 0.88 ms; 0.78M at fan-in 16,
 // 77 tokens, 1000 inputs 731 -> 535 us; 2M, 200 tokens, 8000 inputs 3.00 -> 1.96 ms; 12.6M, 256
-// tokens, 4096 inputs 11.3 -> 10.6 ms (there the 103 GB of row reads bound it: 9.8 TB/s).
+// tokens, 4096 inputs 11.3 -> 10.6 ms (there the 103 GB of row reads bound it: 9.7 TB/s, 58% of the
+// requests past the L2).
 template <int K, int T, bool FLAT>
 __global__ void __launch_bounds__(64) dx_dense_kernel(DxK p, const float* __restrict__ dz) {
   const int lane = threadIdx.x;
@@ -1498,8 +1500,9 @@ constexpr int bwd_waves(int K) { return K == 8 ? 12 : 8; }
 #ifndef BWD_FM_RA
 #define BWD_FM_RA 1
 #endif
-// kept bits with pool windows: waves per workgroup and read-ahead (12 waves: 132 VGPRs, where 16
-// waves held to 128 spilled 20 bytes per lane; C3 dW 19.6 -> 18.9 ms)
+// kept bits with pool windows: waves per workgroup and read-ahead (16 waves leave 128 VGPRs: with bf16
+// windows, 154 at 12 waves, they spill 96 bytes per lane, and 25M neurons, 256 tokens in 256-wide
+// windows take 16.2 ms forward and backward against 12.1; with fp32 windows, 128 either way, even)
 #ifndef BWD_FM_WIN_WAVES
 #define BWD_FM_WIN_WAVES 12
 #endif
@@ -1873,7 +1876,7 @@ extern "C" int gl_bwd(const GlBwdArgs* a, void* stream) {
     // (16 waves with the forward's ReLU bits, else bwd_waves)
     const int dw_waves = a->relu_mask && a->K == 8 ? BWD_FM_WIN_WAVES : q.waves;
     // bf16 X staged in pool windows keeps its bf16 values (8-byte inputs, windows from an even input),
-    // as the forward's windows do: with the forward's ReLU bits (159 VGPRs) or identity neurons;
+    // as the forward's windows do: with the forward's ReLU bits (154 VGPRs) or identity neurons;
     // the ReLU recompute at 12 waves would spill 60 bytes per lane, and keeps fp32 windows
     const bool xbw = dense && a->x_dtype == GL_DTYPE_BF16 && a->D % 2 == 0 && a->D <= 2 * XTILE_DB &&
                      (a->relu_mask || a->act == GL_ACT_IDENTITY);

@@ -238,7 +238,8 @@ struct WinLayout {
 // Narrow layers stage whole token tiles the same way: with win null the "window" is the tile (lo = 0,
 // ww = D, one for every pool), and a stage is tps tiles, contiguous in memory.  tps is the largest
 // power of two (at most 8, the tiles of a mask word) whose tiles fit a region of `slots` 16-byte
-// slots, and no more than a pass has tiles; 0 when not even one tile fits.
+// slots, or the smallest that covers the pass's n_tiles if that is less (4 for 3 tiles: dma_stage
+// copies only tiles that are there); 0 when not even one tile fits.
 inline int stage_tiles(int D, int in_bytes, int slots, int n_tiles) {
   int tps = 0;
   for (int t = 1; t <= 8 && (long long)t * D * in_bytes <= (long long)slots * 16; t *= 2) {

@@ -1241,8 +1241,8 @@ constexpr int fwd_waves(int K, int pk = PK_SUM, int act = GL_ACT_RELU) {
 // 244-256 VGPRs) where 128 KiB of buffers leave one wave per SIMD and nothing to hide its latency.
 // 1M neurons: LogMeanExp, 200 tokens, D = 1500 549 -> 418 us; top-8, 64 tokens, D = 500 264 -> 186;
 // power mean, p = 2, 64 tokens, D = 700 193 -> 145; 0.78M softmax-weighted, 77 tokens, D = 1000 216 -> 150.
-// GELU neurons, max, p = 8 and a p read at run time spill 2-200 VGPRs at 256 and keep the two buffers
-// (max 778 -> 975 us).
+// Top-k spills 11 VGPRs at 256 and gains all the same; GELU neurons, max, p = 8 and a p read at run time
+// spill 2-200 there and keep the two buffers (max 778 -> 975 us).
 constexpr bool fwd_narrow16(int K, int pk, int act) {
   return K == 16 && act != GL_ACT_GELU && (pk == PK_LME || pk == PK_SW || pk == PK_TOPK || (pk_pint(pk) > 0 && pk_pint(pk) < 8));
 }

@@ -7,13 +7,16 @@
 // each gathered value of X serves 16 neurons, where the per-neuron kernels gather it 16 times.
 //
 // X lies in slices of 64 tokens, [slice][input][64 tokens] fp32: an input of a slice is one 256-byte
-// row (a slice of 4096 inputs is 1 MiB, so the slices in use stay in an XCD's L2), and a wave loads
-// the 16 rows of a record with four 1-KiB loads straight into MFMA operands, with no LDS.
+// row, and a wave loads the 16 rows of a record with four 1-KiB loads straight into the forward's MFMA
+// operands (dW takes them again transposed, through LDS).  A slice of 4096 inputs is 1 MiB, so the
+// slices in use stay in an XCD's L2; one of 65,536 is 16 MiB and does not, which costs 20% (4.2M neurons,
+// 64 tokens: forward 158 us at 4096 inputs, 189 at 65,536; the per-neuron kernels 351 and 536).
 //
 // Bounds: at 12.6M neurons, 512 tokens, 4096 inputs the forward runs 2.17 ms and the dW pass 4.85 ms
 // (7.47 and 10.5 in the per-neuron kernels; the products alone take 1.31 and 2.62 ms at the 157 TFLOP/s
-// of fp32 MFMA).  Beside the MFMAs the forward issues 32 VALU per record and slice (the activation and
-// the sum), the dW pass ~110 (dz, mask bits, db).  The second layout of X that dW needs (inputs, not
+// of fp32 MFMA).  Counted beside the MFMAs: 61 VALU per record and slice in the forward (0.62 ms of issue),
+// 93 in the dW pass (0.95: dz, mask bits, db).  The dW pass with ReLU holds 224 VGPRs (2 waves per SIMD)
+// and spills 44 SGPRs to VGPR lanes.  The second layout of X that dW needs (inputs, not
 // tokens, across lanes) read again from memory ran 5.70 ms (4.69 then): 16-byte pieces of 64 rows per load, and
 // the rows no longer in the 32-KiB L1.  Loads, not LDS, feed the products because a slice of 64
 // tokens of a wide layer (1 MiB) fits no LDS, while 4 tokens (what does fit) leave 3/4 of a tile idle.
@@ -211,7 +214,8 @@ struct RecBwdK {
 // D holds tokens 16 G + 4 q + i of neuron m.  dz = c1 [z > 0] is then already the B operand of
 // dW^T[k][neuron] += sum over tokens X^T[k][token] dz[token][neuron] (k-slot G = token 16 G + 4 q + i),
 // whose A operand, input m of the record at those tokens, comes from the same rows through a
-// transpose in the wave's own LDS (rows of 68 floats: the reads of 16 rows hit 16 residues).  Per slice a lane's 16 mask bits are 16 consecutive tokens of its neuron: one 16-bit store.
+// transpose in the wave's own LDS (rows of 68 floats: the reads of 16 rows hit 16 residues).  Per slice
+// a lane's 16 mask bits are 16 consecutive tokens of its neuron: one 16-bit store.
 constexpr int REC_XROW = 68;
 template <int ACT>
 __global__ void __launch_bounds__(REC_WAVES * 64, 2) rec_bwd_w_kernel(RecBwdK p) {
